@@ -5,8 +5,8 @@
 //                     (radix_ops.decode_bits, radix_kernel_gpu.py:614-636)
 //   k_schedule        the per-block tier stream lengths
 //                     (radix_ops.prepare_schedule, radix_kernel_gpu.py:44-66)
-//   k_gemv_generic    decode + GEMV for any widths, block size, ragged rows,
-//                     M = 1..8 (radix_ops.gemv_fused / gemv_mc,
+//   k_gemv_generic    decode + GEMV for any widths and block size, M = 1..8
+//                     (radix_ops.gemv_fused / gemv_mc,
 //                     radix_kernel_gpu.py:682-718, radix_ops.py:91-164)
 //   k_gemv_sip        the fused decode + GEMV for sip (3, 8) streams over
 //                     whole 1024-weight blocks and M = 1..8 bf16 activation
@@ -19,6 +19,10 @@
 //   k_gemv_gulp       the same for gulp (2, 2, 4, 8) streams
 //                     (radix_kernel_gpu.py:292-392); M = 8 in quad units; a
 //                     decode mode
+//   k_gemv_wave, k_decode_wave (wave_kernels.h)
+//                     the GEMV and the decode of 1024-weight blocks the
+//                     sip and gulp kernels do not take: ragged columns, the
+//                     balanced profile, fp32 activations
 //   k_gemv_narrow     a raw row-major bf16 weight against M <= 8 rows
 //                     (radix_ops.gemv_narrow, radix_ops.py:177-249)
 //
@@ -1872,6 +1876,10 @@ void k_gemv_gulp(const SipGroup g, const uint16_t* __restrict__ x, const SipShap
     }
 }
 
+// ------------------------------- ragged columns, balanced, fp32 activations --
+
+#include "wave_kernels.h"
+
 // ------------------------------------------------------ raw bf16 GEMV --
 //
 // drinkme's _gemv_narrow (src/drinkme/codec/radix_ops.py:177-249), the
@@ -2292,6 +2300,69 @@ int launch_gulp(const dmx_radix_tensor* const* ts, uint32_t n, const void* x, ui
     return launch_check(err, errn, "gulp gemv launch");
 }
 
+typedef void (*WaveKernel)(const WaveGroup, const void*, const WaveShape);
+
+// k_gemv_wave for profile p, M = 1, 2, 4, 8 (mi 0..3) and the activation type
+template <int P>
+WaveKernel wave_kernel_of(int mi, int xt) {
+    static const WaveKernel table[2][4] = {
+        {k_gemv_wave<P, 1, kWaveX16>, k_gemv_wave<P, 2, kWaveX16>, k_gemv_wave<P, 4, kWaveX16>,
+         k_gemv_wave<P, 8, kWaveX16>},
+        {k_gemv_wave<P, 1, kWaveX32>, k_gemv_wave<P, 2, kWaveX32>, k_gemv_wave<P, 4, kWaveX32>,
+         k_gemv_wave<P, 8, kWaveX32>}};
+    return table[xt][mi];
+}
+WaveKernel wave_kernel(int p, int mi, int xt) {
+    return p == kWaveSip        ? wave_kernel_of<kWaveSip>(mi, xt)
+           : p == kWaveBalanced ? wave_kernel_of<kWaveBalanced>(mi, xt)
+           : p == kWaveGulp     ? wave_kernel_of<kWaveGulp>(mi, xt)
+                                : wave_kernel_of<kWaveRaw>(mi, xt);
+}
+
+// The profile whose wave kernel takes tensor t, or -1.
+int wave_takes(const dmx_radix_tensor* t) {
+    return fast_policy() && t->block_size == 1024 && fast_directory(t) ? wave_profile(t->n_widths, t->widths) : -1;
+}
+
+// One launch of the wave kernel over n tensors of profile p and equal cols
+// (already checked; kWaveRaw: t->data is the raw weight). Returns 2, having
+// launched nothing, when two rows' sums per column block do not fit the LDS.
+int launch_wave(int p, const dmx_radix_tensor* const* ts, uint32_t n, const void* x, int x_dtype, uint32_t m,
+                const void* const* bias, int bias_dtype, void* const* out, int out_dtype, hipStream_t stream, char* err,
+                size_t errn) {
+    if (n < 1 || n > (uint32_t)kGroupMax || m < 1 || m > 8) return 2;
+    const int mi = m == 1 ? 0 : m == 2 ? 1 : m <= 4 ? 2 : 3, xt = x_dtype == DMX_BF16 ? kWaveX16 : kWaveX32;
+    WaveShape sh;
+    sh.cols = ts[0]->cols;
+    sh.nb = (sh.cols + 1023) / 1024;
+    sh.m = m;
+    sh.x_dtype = x_dtype;
+    sh.bias_dtype = bias_dtype;
+    sh.out_dtype = out_dtype;
+    sh.wide = xt == kWaveX32 || (sh.cols % 2 == 0 && reinterpret_cast<uintptr_t>(x) % 4 == 0);
+    uint64_t rows = 0;
+    for (uint32_t i = 0; i < n; ++i) rows += ts[i]->rows;
+    const uint32_t M = 1u << mi, W = wave_waves(p, (int)M, xt);
+    sh.tile = wave_tile(rows, sh.nb, M, (uint32_t)cu_count() * wave_occ(p, (int)M, xt) * 4u / W, wave_lds(p, W));
+    if (sh.tile == 0) return 2;
+    WaveGroup g;
+    uint64_t wgs = 0;
+    for (uint32_t i = 0; i < (uint32_t)kGroupMax; ++i) {
+        const uint32_t k = i < n ? i : n - 1;
+        g.data[i] = ts[k]->data;
+        g.offsets[i] = ts[k]->offsets;
+        g.palette[i] = ts[k]->palette;
+        g.bias[i] = bias ? bias[k] : nullptr;
+        g.out[i] = out[k];
+        g.rows[i] = ts[k]->rows;
+        g.wg0[i] = i < n ? (uint32_t)wgs : ~0u;
+        if (i < n) wgs += (ts[i]->rows + sh.tile - 1) / sh.tile;
+        if (wgs >= (1ull << 31)) return 2;
+    }
+    hipLaunchKernelGGL(wave_kernel(p, mi, xt), dim3((uint32_t)wgs), dim3(W * 64), sh.tile * sh.nb * M * 4, stream, g, x, sh);
+    return launch_check(err, errn, "wave gemv launch");
+}
+
 template <int M, bool RAW = false>
 void launch_generic_m(const Desc& d, const void* x, int x_dtype, const void* bias, int bias_dtype, void* out,
                       int out_dtype, hipStream_t stream) {
@@ -2317,6 +2388,11 @@ int gemv_one(const dmx_radix_tensor* t, const Desc& d, const void* x, int x_dtyp
     }
     if (gulp_eligible(t, x, x_dtype, m)) {
         const int rc = launch_gulp(&t, 1, x, m, &bias, bias_dtype, &out, out_dtype, s, err, errn);
+        if (rc != 2) return rc;
+    }
+    const int p = wave_takes(t);
+    if (p >= 0) {
+        const int rc = launch_wave(p, &t, 1, x, x_dtype, m, &bias, bias_dtype, &out, out_dtype, s, err, errn);
         if (rc != 2) return rc;
     }
     switch (m) {
@@ -2414,6 +2490,18 @@ extern "C" int dmx_radix_decode(const dmx_radix_tensor* t, uint16_t* out, void* 
     if (!out) return fail(err, errn, "null output");
     const int rc = launch_decode_fast(t, out, static_cast<hipStream_t>(stream), err, errn);
     if (rc != 2) return rc;
+    const int p = wave_takes(t);
+    if (p >= 0) {
+        typedef void (*Kernel)(Desc, uint16_t*, uint32_t, uint32_t);
+        const Kernel kern = p == kWaveSip ? k_decode_wave<kWaveSip>
+                            : p == kWaveBalanced ? k_decode_wave<kWaveBalanced> : k_decode_wave<kWaveGulp>;
+        const uint32_t blocks = d.rows * d.nb, waves = (uint32_t)cu_count() * 2 * kDecodeWaves;
+        const uint32_t run = std::min<uint32_t>(64, (blocks + waves - 1) / waves), per_wg = run * kDecodeWaves;
+        const uint32_t wide = d.cols % 2 == 0 && reinterpret_cast<uintptr_t>(out) % 4 == 0;
+        hipLaunchKernelGGL(kern, dim3((blocks + per_wg - 1) / per_wg), dim3(kDecodeWaves * 64), 0,
+                           static_cast<hipStream_t>(stream), d, out, run, wide);
+        return launch_check(err, errn, "wave decode launch");
+    }
     hipLaunchKernelGGL(k_decode, dim3(d.rows * d.nb), dim3(kGenThreads), 0, static_cast<hipStream_t>(stream), d, out);
     return launch_check(err, errn, "decode launch");
 }
@@ -2443,6 +2531,7 @@ extern "C" int dmx_radix_gemv_group(const dmx_radix_tensor* const* tensors, uint
     if (!tensors || !out || n == 0) return fail(err, errn, "empty tensor group");
     Desc d[kGroupMax];
     bool all_sip = n <= (uint32_t)kGroupMax, all_gulp = all_sip;
+    int wave = all_sip ? wave_takes(tensors[0]) : -1;  // the profile they share, none taken by the sip or gulp kernel
     for (uint32_t i = 0; i < n; ++i) {
         Desc di;
         if (check_tensor(tensors[i], di, err, errn)) return 1;
@@ -2451,6 +2540,9 @@ extern "C" int dmx_radix_gemv_group(const dmx_radix_tensor* const* tensors, uint
             return 1;
         all_sip = all_sip && sip_eligible(tensors[i], x, x_dtype, m);
         all_gulp = all_gulp && gulp_eligible(tensors[i], x, x_dtype, m);
+        if (sip_eligible(tensors[i], x, x_dtype, m) || gulp_eligible(tensors[i], x, x_dtype, m) ||
+            wave_takes(tensors[i]) != wave)
+            wave = -1;
         if (i < (uint32_t)kGroupMax) d[i] = di;
     }
     hipStream_t s = static_cast<hipStream_t>(stream);
@@ -2460,6 +2552,10 @@ extern "C" int dmx_radix_gemv_group(const dmx_radix_tensor* const* tensors, uint
     }
     if (all_gulp) {
         const int rc = launch_gulp(tensors, n, x, m, bias, bias_dtype, out, out_dtype, s, err, errn);
+        if (rc != 2) return rc;
+    }
+    if (wave >= 0) {
+        const int rc = launch_wave(wave, tensors, n, x, x_dtype, m, bias, bias_dtype, out, out_dtype, s, err, errn);
         if (rc != 2) return rc;
     }
     for (uint32_t i = 0; i < n; ++i) {
@@ -2599,6 +2695,12 @@ extern "C" int dmx_radix_gemv_twin(const uint16_t* w, uint32_t rows, uint32_t co
                       (reinterpret_cast<uintptr_t>(w) & 15u) == 0;
     if (fast && (is_sip(&t) || is_gulp(&t))) {
         const int rc = launch_raw(w, rows, cols, is_gulp(&t), x, m, bias, bias_dtype, out, out_dtype, s, err, errn);
+        if (rc != 2) return rc;
+    }
+    if (wave_takes(&t) >= 0) {
+        t.data = reinterpret_cast<const uint32_t*>(w);
+        const dmx_radix_tensor* tp = &t;
+        const int rc = launch_wave(kWaveRaw, &tp, 1, x, x_dtype, m, &bias, bias_dtype, &out, out_dtype, s, err, errn);
         if (rc != 2) return rc;
     }
     Desc d = {};

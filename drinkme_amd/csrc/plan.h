@@ -566,4 +566,17 @@ inline bool plan_gulp(SipShape& sh, const uint32_t* row0, uint32_t n, uint32_t m
     return true;
 }
 
+// The wave kernel's rows per workgroup T: even, enough that the group's rows
+// make about `slots` workgroups, the ones the chip holds at once, and no
+// more than keep a tile's sums (one float per row, column block and
+// activation row) to 16 KB, and with the kernel's static LDS `fixed` to 64
+// KB, so two workgroups fit a CU. 0: not even two rows fit.
+constexpr size_t kWaveSums = 16 * 1024;
+inline uint32_t wave_tile(uint64_t rows, uint32_t nb, uint32_t M, uint32_t slots, size_t fixed) {
+    const uint64_t row_bytes = (uint64_t)nb * M * 4;
+    const uint64_t most = std::min(kWaveSums, 64 * 1024 - fixed) / row_bytes & ~1ull;
+    const uint64_t even = ((rows + slots - 1) / slots + 1) & ~1ull;
+    return (uint32_t)std::min(most, std::max<uint64_t>(even, 2));
+}
+
 }  // namespace dmx

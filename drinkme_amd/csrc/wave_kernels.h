@@ -1,0 +1,795 @@
+// The wave kernels: decode + GEMV (k_gemv_wave) and decode alone
+// (k_decode_wave) for 1024-weight blocks of the three profiles, any column
+// count, any activation type. They serve what the sip and gulp kernels do
+// not take: columns that are not whole blocks, the balanced profile, and
+// fp32 activations. Included by kernels.hip, inside its namespace.
+//
+// Work split. A workgroup of W waves owns T rows (T even) of one tensor. A
+// unit is one column block of two neighbouring rows; the units, column by
+// column, are dealt to the waves in contiguous runs. So a wave stays on one
+// column block for a run of rows and keeps that block's activations in
+// registers, 16 columns a lane: they are read once per column block (from
+// L2), not once per weight block, and cost no LDS traffic at any M. Each
+// weight block's M sums are reduced over the lanes (both rows of the unit
+// at once) into LDS, and a row's column blocks are added in order at the
+// end. Every sum is a function of the row and the activation alone: the
+// same for any M, T and W.
+//
+// What bounds it: VALU issue (80% busy between a launch's start and end: 91
+// VALU instructions a sip block, 106 a balanced one at M = 1 bf16, 16 M + 16
+// more for the fp32 products), then the 3 us of a launch before and after
+// its blocks. Measured, one launch, against k_gemv_generic, which scans
+// over a workgroup with two barriers a tier: sip 2 x 9472 x 3584 (ragged)
+// 24.5 us for 284, sip 3584 x 9472 15.8 for 149; gulp fp32 M = 2 q/k/v of
+// 10240 x 5120 31.4 for 326; balanced q/k/v of 6144 x 4096 16.0 for 145.
+//
+// The decode works on bytes. A table entry holds four exponent bytes and a
+// v_perm selector over (four consecutive bytes of the next tier's
+// exponents, the entry's own four): byte k is k where weight k resolved in
+// this tier, 4 + its rank among the group's escapes where it did not. One
+// v_perm so completes a group, and bit 2 of a selector byte is the escape
+// flag, which a masked popcount counts.
+//   tier 0   lane l owns weights 16l .. 16l + 15, four table lookups;
+//   tier 1   (balanced, gulp) lane l resolves the block's tier-0 escapes
+//            8l .. 8l + 7 from the tail words, which a wave keeps in LDS,
+//            and writes their exponent bytes, in order, to LDS;
+//   tier 2   (gulp) lane l resolves the tier-1 escapes 2l, 2l + 1 so;
+//   terminal raw exponent bytes, read in place from the tail words.
+// Each level reads the four bytes at its first escape's rank from the level
+// below (two LDS words and a funnel shift). The ranks come from one DPP scan
+// a level for both rows of a unit (counts of at most 1024, 16 bits each).
+// The two rows' decodes run side by side with no branch between them, so one
+// row's LDS round trips cover the other's (decoded one after the other, the
+// waves waited 44% of their time). A unit with a block outside the limits
+// (more than 512 tier-0 or 128 tier-1 escapes, a tail of more than 64
+// words, streams cut short) takes wave_exact, which reads every field from
+// memory as decode_block does.
+
+enum WaveProfile { kWaveSip = 0, kWaveBalanced = 1, kWaveGulp = 2, kWaveRaw = 3 };
+
+// Profile of a tensor's widths, or -1.
+inline int wave_profile(uint32_t n_widths, const uint32_t* w) {
+    if (n_widths == 2 && w[0] == 3 && w[1] == 8) return kWaveSip;
+    if (n_widths == 3 && w[0] == 2 && w[1] == 3 && w[2] == 8) return kWaveBalanced;
+    if (n_widths == 4 && w[0] == 2 && w[1] == 2 && w[2] == 4 && w[3] == 8) return kWaveGulp;
+    return -1;
+}
+
+constexpr uint32_t wave_tiers(int P) { return P == kWaveSip ? 1u : P == kWaveBalanced ? 2u : 3u; }  // nonterminal
+constexpr uint32_t wave_width(int P, uint32_t j) {
+    return P == kWaveSip ? 3u : j == 0 ? 2u : P == kWaveBalanced ? 3u : j == 1 ? 2u : 4u;
+}
+// byte offset of tier j's run in the padded palette tables
+constexpr uint32_t wave_pal_byte(int P, uint32_t j) {
+    uint32_t b = 0;
+    for (uint32_t k = 0; k < j; ++k) b += 1u << wave_width(P, k);
+    return b;
+}
+
+// The activation types of the wave kernel, its element reads and stores.
+constexpr int kWaveX16 = 0, kWaveX32 = 1;
+
+struct WaveTables {
+    // entries of kWaveSip: 4096 (four 3-bit codes); balanced: 256 (four 2-bit
+    // codes) then 4096; gulp: 256, 256 (four 2-bit codes each) and 256 (two
+    // 4-bit codes)
+    static constexpr uint32_t entries(int P) {
+        return P == kWaveSip ? 4096u : P == kWaveBalanced ? 256u + 4096u : P == kWaveGulp ? 768u : 1u;
+    }
+    static constexpr uint32_t tier(int P, uint32_t j) { return j == 0 ? 0u : j == 1 ? 256u : 512u; }
+};
+
+// A wave's LDS exchange, in words, per row of a unit: the tail words and one
+// more, the tier-1 exponent bytes (512 and a window's overhang) and the
+// tier-2 ones (128 and the overhang).
+constexpr uint32_t kExTail = 0, kExT1 = 66, kExT2 = kExT1 + 130;
+constexpr uint32_t wave_exchange(int P) {
+    return P == kWaveSip ? kExT1 : P == kWaveBalanced ? kExT2 : P == kWaveGulp ? kExT2 + 34 : 0u;
+}
+
+// Four bytes at byte address `at` of LDS words: the two words holding them
+// and a funnel shift. (One unaligned ds_read_b32 instead stalls the LDS for
+// about 60 cycles a wave: the 9472 x 3584 gate/up launch took 45.6 us with
+// it, 28.8 us without.)
+__device__ __forceinline__ uint32_t lds_bytes(const uint32_t* words, uint32_t at) {
+    const uint32_t* p = reinterpret_cast<const uint32_t*>(reinterpret_cast<const uint8_t*>(words) + (at & ~3u));
+    return __builtin_amdgcn_alignbyte(p[1], p[0], at);
+}
+
+// Entry of four codes c[k] < 2^w, exponents from the run `pal` of the padded
+// tables (the escape code reads its zero pad byte).
+template <uint32_t w, uint32_t N>
+__device__ __forceinline__ uint2 wave_entry(uint32_t i, const uint32_t (&pal)[4]) {
+    uint32_t e = 0, sel = 0x03020100u, r = 4;
+#pragma unroll
+    for (uint32_t k = 0; k < N; ++k) {
+        const uint32_t c = (i >> (w * k)) & ((1u << w) - 1u);
+        uint32_t b = __builtin_amdgcn_perm(pal[1], pal[0], c & 7u);
+        if (w == 4) b = c & 8u ? __builtin_amdgcn_perm(pal[3], pal[2], c & 7u) : b;
+        e |= (b & 0xFFu) << (8 * k);
+        if (c == (1u << w) - 1u) sel ^= (k ^ r++) << (8 * k);
+    }
+    return make_uint2(e, sel);
+}
+
+// The 4096 entries of four 3-bit codes (palette words p0, p1): entries 8h ..
+// 8h + 7 share the upper three codes, and only c0 = 7 (an escape) moves
+// their ranks.
+__device__ __forceinline__ void wave_table3(uint2* tab, uint32_t p0, uint32_t p1, uint32_t threads) {
+    const uint32_t pal[4] = {p0, p1, 0, 0};
+    for (uint32_t h = threadIdx.x; h < 512; h += threads) {
+        const uint2 e = wave_entry<3, 4>(8 * h, pal), esc = wave_entry<3, 4>(8 * h + 7, pal);
+        const uint32_t up = e.x & 0xFFFFFF00u;
+#pragma unroll
+        for (uint32_t c = 0; c < 8; c += 2) {
+            const uint32_t two = c < 4 ? p0 >> (8 * c) : p1 >> (8 * (c - 4));
+            const uint2 odd = c == 6 ? esc : make_uint2(up | ((two >> 8) & 0xFFu), e.y);
+            *reinterpret_cast<uint4*>(tab + 8 * h + c) = make_uint4(up | (two & 0xFFu), e.y, odd.x, odd.y);
+        }
+    }
+}
+
+// Builds the tables of profile P (all of the workgroup's threads).
+template <int P>
+__device__ __forceinline__ void wave_tables(uint2* tab, const uint32_t* palette, uint32_t threads) {
+    const const_u32_ptr p = (const_u32_ptr)palette;
+    if constexpr (P == kWaveSip) {
+        wave_table3(tab, p[0], p[1], threads);
+    } else if constexpr (P == kWaveBalanced) {
+        const uint32_t pal0[4] = {p[0], 0, 0, 0};
+        for (uint32_t i = threadIdx.x; i < 256; i += threads) tab[i] = wave_entry<2, 4>(i, pal0);
+        wave_table3(tab + 256, p[1], p[2], threads);
+    } else if constexpr (P == kWaveGulp) {
+        const uint32_t pal0[4] = {p[0], 0, 0, 0}, pal1[4] = {p[1], 0, 0, 0}, pal2[4] = {p[2], p[3], p[4], p[5]};
+        for (uint32_t i = threadIdx.x; i < 768; i += threads)
+            tab[i] = i < 256 ? wave_entry<2, 4>(i, pal0) : i < 512 ? wave_entry<2, 4>(i - 256, pal1)
+                                                                  : wave_entry<4, 2>(i - 512, pal2);
+    }
+}
+
+// A block's loads: the lane's 16 literal bytes, its tier-0 codes and its
+// tail word (the streams after tier 0).
+struct WaveStage {
+    u32x4 lit;
+    u32x2 t0;
+    uint32_t tail;
+};
+
+__device__ __forceinline__ uint32_t block_fixed(int P, uint32_t n) { return words_for(n, 8) + words_for(n, wave_width(P, 0)); }
+
+// Loads block [start, end) of n weights, non-temporal, through a buffer
+// resource that ends four words past the block (or its fixed streams, where
+// the block is cut shorter than those): no wide load of a lane straddles the
+// end, and those words are the next block's or the pad's. The tail's lanes
+// past the block take an offset past the resource: they read 0 and fetch
+// nothing. live = false: nothing is fetched. The loads are unconditional, so
+// the compiler's waits for one stage leave the next one's loads in flight.
+template <int P>
+__device__ __forceinline__ WaveStage wave_load(const uint32_t* data, uint32_t start, uint32_t end, uint32_t n, bool live,
+                                               uint32_t lane) {
+    const int32_t len = (int32_t)(end - start);
+    const uint32_t lw = words_for(n, 8), fixed = block_fixed(P, n);
+    const uint32_t reach = 4u * ((uint32_t)max(len, (int32_t)fixed) + 4u);
+    const auto r = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint32_t*>(data + start), 0, live ? reach : 0u, 0x00020000);
+    constexpr int nt = 2;
+    WaveStage s;
+    s.lit = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, 16 * lane, 0, nt));
+    if constexpr (P == kWaveSip) {
+        s.t0 = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(r, 4 * (lw + ((3 * lane) >> 1)), 0, nt));
+    } else {
+        s.t0.x = __builtin_amdgcn_raw_buffer_load_b32(r, 4 * (lw + lane), 0, nt);
+        s.t0.y = 0;
+    }
+    s.tail = __builtin_amdgcn_raw_buffer_load_b32(
+        r, (int32_t)lane < len - (int32_t)fixed ? 4 * (fixed + lane) : 0x80000000u, 0, nt);
+    return s;
+}
+
+// The lane's 16 exponent bytes with every field read from memory, as
+// decode_block reads them (any escape counts, streams of any length).
+template <int P>
+__device__ void wave_exact(const uint32_t* data, const uint8_t* pal, uint32_t start, uint32_t end, uint32_t n,
+                           uint32_t lane, uint32_t (&E)[4]) {
+    const uint32_t valid = n > 16 * lane ? min(16u, n - 16 * lane) : 0u;
+    uint32_t active = (1u << valid) - 1u;
+    uint64_t elo = 0, ehi = 0;  // exponent byte of weight i: byte i & 7 of (i < 8 ? elo : ehi)
+    auto place = [&](int i, uint32_t e) {
+        const uint64_t v = (uint64_t)e << (8 * (i & 7));
+        if (i < 8)
+            elo |= v;
+        else
+            ehi |= v;
+    };
+    uint32_t pos = start + words_for(n, 8);
+#pragma unroll
+    for (uint32_t j = 0; j < wave_tiers(P); ++j) {
+        const uint32_t w = wave_width(P, j), esc = (1u << w) - 1u;
+        const uint32_t cnt = __builtin_popcount(active), inc = wave_scan_incl(cnt);
+        uint32_t r = inc - cnt;
+#pragma unroll 1
+        for (int i = 0; i < 16; ++i) {
+            if (!((active >> i) & 1u)) continue;
+            const uint32_t code = field(data + pos, r++, w);
+            if (code == esc) continue;
+            place(i, pal[wave_pal_byte(P, j) + code]);
+            active &= ~(1u << i);
+        }
+        pos += words_for(__builtin_amdgcn_readlane(inc, 63), w);
+    }
+    const uint32_t cnt = __builtin_popcount(active), inc = wave_scan_incl(cnt);
+    uint32_t r = inc - cnt;
+    if (end > pos) {  // (the terminal is read only where the directory gives the block words for it)
+#pragma unroll 1
+        for (int i = 0; i < 16; ++i)
+            if ((active >> i) & 1u) place(i, field(data + pos, r++, 8));
+    }
+    E[0] = (uint32_t)elo;
+    E[1] = (uint32_t)(elo >> 32);
+    E[2] = (uint32_t)ehi;
+    E[3] = (uint32_t)(ehi >> 32);
+}
+
+// The first `bits` (clamped to 0 .. most < 32) bits of codes: those past the
+// stream's end read as 0, which no tier takes for an escape.
+__device__ __forceinline__ uint32_t keep_bits(uint32_t codes, int32_t bits, int32_t most) {
+    return __builtin_amdgcn_ubfe(codes, 0, (uint32_t)min(max(bits, 0), most));
+}
+
+// Escapes of an entry, added to n.
+__device__ __forceinline__ uint32_t add_escapes(uint2 e, uint32_t n) {
+    return (uint32_t)__builtin_popcount(e.y & 0x04040404u) + n;
+}
+
+// Completes an entry from the next tier's exponent bytes (at byte `at` of
+// `bytes`, the group's first escape).
+__device__ __forceinline__ uint32_t complete(uint2 e, const uint32_t* bytes, uint32_t at) {
+    return __builtin_amdgcn_perm(lds_bytes(bytes, at), e.x, e.y);
+}
+
+// Decodes R blocks of n weights (R = 2: a unit's rows; 1) from their loaded
+// stages: hi[j][g], lo[j][g] = the high and low bytes of the bf16 bits of the
+// lane's weights 4g .. 4g + 3 of block j (weight k in byte k). Weights past n
+// get exponent 0 (a zero or denormal, finite: their activations are 0). ex:
+// the wave's exchange, R x wave_exchange(P) words, in front of the tables, so
+// that a block outside the limits, whose window addresses reach at most 1 KB
+// too far, still reads inside the LDS array.
+template <int P, int R>
+__device__ __forceinline__ void wave_decode(const uint2* tab, uint32_t* ex, const WaveStage (&s)[R], const uint32_t* data,
+                                            const uint8_t* pal, const uint32_t (&start)[R], const uint32_t (&end)[R],
+                                            uint32_t n, uint32_t lane, uint32_t (&hi)[R][4], uint32_t (&lo)[R][4]) {
+    constexpr uint32_t stride = wave_exchange(P);
+    const uint32_t fixed = block_fixed(P, n);
+    uint2 e[R][4];
+    uint32_t c[R][4];  // escapes of groups 0 .. g
+    int32_t tail[R], bad = 0;  // (bad: negative once a limit is passed; every quantity is far below 2^31)
+    uint32_t T[R][2];
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+        tail[j] = (int32_t)(end[j] - start[j] - fixed);
+        bad |= 64 - tail[j];
+        ex[j * stride + kExTail + lane] = s[j].tail;
+        if constexpr (P == kWaveSip) {
+            const uint64_t v = ((uint64_t)s[j].t0.y << 32 | s[j].t0.x) >> ((lane & 1) * 16);
+            T[j][0] = (uint32_t)v;
+            T[j][1] = (uint32_t)(v >> 32);
+        } else {
+            T[j][0] = s[j].t0.x;
+        }
+    }
+    if (n < 1024) {
+        const int32_t bits = ((int32_t)n - 16 * (int32_t)lane) * (int32_t)wave_width(P, 0);
+#pragma unroll
+        for (int j = 0; j < R; ++j) {
+            T[j][0] = bits >= 32 ? T[j][0] : keep_bits(T[j][0], bits, 31);
+            if constexpr (P == kWaveSip) T[j][1] = keep_bits(T[j][1], bits - 32, 16);
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+        if constexpr (P == kWaveSip) {
+            e[j][0] = tab[T[j][0] & 0xFFFu];
+            e[j][1] = tab[(T[j][0] >> 12) & 0xFFFu];
+            e[j][2] = tab[__builtin_amdgcn_alignbit(T[j][1], T[j][0], 24) & 0xFFFu];
+            e[j][3] = tab[(T[j][1] >> 4) & 0xFFFu];
+        } else {
+#pragma unroll
+            for (int g = 0; g < 4; ++g) e[j][g] = tab[(T[j][0] >> (8 * g)) & 0xFFu];
+        }
+    }
+    // counts of both rows through one scan, row j in bits 16j .. 16j + 15
+    uint32_t q[R], n1[R];
+    auto scan = [&](const uint32_t (&cnt)[R], uint32_t (&first)[R], uint32_t (&total)[R]) {
+        const uint32_t v = R == 2 ? cnt[0] | cnt[R - 1] << 16 : cnt[0];
+        const uint32_t inc = wave_scan_incl_dpp(v), x = inc - v, t = __builtin_amdgcn_readlane(inc, 63);
+        first[0] = R == 2 ? x & 0xFFFFu : x;
+        total[0] = R == 2 ? t & 0xFFFFu : t;
+        if (R == 2) {
+            first[R - 1] = x >> 16;
+            total[R - 1] = t >> 16;
+        }
+    };
+    uint32_t cnt[R];
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+        c[j][0] = add_escapes(e[j][0], 0);
+#pragma unroll
+        for (int g = 1; g < 4; ++g) c[j][g] = add_escapes(e[j][g], c[j][g - 1]);
+        cnt[j] = c[j][3];
+    }
+    scan(cnt, q, n1);
+    uint32_t bytes = kExTail;  // where tier 0's escapes lie, in words of the exchange
+    if constexpr (P == kWaveSip) {
+#pragma unroll
+        for (int j = 0; j < R; ++j) bad |= 4 * tail[j] - (int32_t)n1[j];
+    } else {
+        // lane l: the block's tier-1 codes 8l .. 8l + 7
+        constexpr uint32_t w = wave_width(P, 1);
+        uint32_t w1[R], g0[R], q1[R], n2[R];
+        uint2 a[R][2];
+#pragma unroll
+        for (int j = 0; j < R; ++j) {
+            const uint32_t* t = ex + j * stride + kExTail;
+            w1[j] = words_for(n1[j], w);
+            const int32_t bits = (int32_t)(w * n1[j]) - (int32_t)(8 * w * lane);
+            if constexpr (P == kWaveBalanced) {
+                const uint32_t code = keep_bits(lds_bytes(t, 3 * lane), bits, 24);
+                a[j][0] = tab[256 + (code & 0xFFFu)];
+                a[j][1] = tab[256 + (code >> 12)];
+            } else {
+                const uint32_t code = keep_bits(reinterpret_cast<const uint16_t*>(t)[lane], bits, 16);
+                a[j][0] = tab[256 + (code & 0xFFu)];
+                a[j][1] = tab[256 + (code >> 8)];
+            }
+            g0[j] = add_escapes(a[j][0], 0);
+            cnt[j] = add_escapes(a[j][1], g0[j]);
+        }
+        scan(cnt, q1, n2);
+        if constexpr (P == kWaveBalanced) {
+#pragma unroll
+            for (int j = 0; j < R; ++j) {
+                const int32_t left = tail[j] - (int32_t)w1[j];  // terminal words
+                bad |= (512 - (int32_t)n1[j]) | left | (4 * left - (int32_t)n2[j]);
+                const uint32_t* t = ex + j * stride + kExTail + (w1[j] & 63u);
+                a[j][0].x = complete(a[j][0], t, q1[j]);
+                a[j][1].x = complete(a[j][1], t, q1[j] + g0[j]);
+            }
+        } else {
+            // lane l: the block's tier-2 codes 2l, 2l + 1
+            uint2 b[R];
+            uint32_t w2[R];
+#pragma unroll
+            for (int j = 0; j < R; ++j) {
+                w2[j] = words_for(n2[j], 4);
+                const uint32_t code = reinterpret_cast<const uint8_t*>(ex + j * stride + kExTail + (w1[j] & 63u))[lane];
+                b[j] = tab[512 + keep_bits(code, (int32_t)(4 * n2[j]) - (int32_t)(8 * lane), 8)];
+                cnt[j] = add_escapes(b[j], 0);
+                bad |= (512 - (int32_t)n1[j]) | (128 - (int32_t)n2[j]) | (tail[j] - (int32_t)(w1[j] + w2[j]));
+            }
+            if (__builtin_amdgcn_ballot_w64((cnt[0] | cnt[R - 1]) != 0) != 0) {
+                uint32_t q2[R], n3[R];
+                scan(cnt, q2, n3);
+#pragma unroll
+                for (int j = 0; j < R; ++j) {
+                    bad |= 4 * (tail[j] - (int32_t)(w1[j] + w2[j])) - (int32_t)n3[j];
+                    b[j].x = complete(b[j], ex + j * stride + kExTail + ((w1[j] + w2[j]) & 63u), q2[j]);
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < R; ++j) reinterpret_cast<uint16_t*>(ex + j * stride + kExT2)[lane] = (uint16_t)b[j].x;
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int j = 0; j < R; ++j) {
+                a[j][0].x = complete(a[j][0], ex + j * stride + kExT2, q1[j]);
+                a[j][1].x = complete(a[j][1], ex + j * stride + kExT2, q1[j] + g0[j]);
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < R; ++j)
+            *reinterpret_cast<uint2*>(ex + j * stride + kExT1 + 2 * lane) = make_uint2(a[j][0].x, a[j][1].x);
+        __builtin_amdgcn_wave_barrier();
+        bytes = kExT1;
+    }
+    uint32_t E[R][4];
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+        const uint32_t* t = ex + j * stride + bytes;
+        E[j][0] = complete(e[j][0], t, q[j]);
+#pragma unroll
+        for (int g = 1; g < 4; ++g) E[j][g] = complete(e[j][g], t, q[j] + c[j][g - 1]);
+    }
+    __builtin_amdgcn_wave_barrier();
+    if (__builtin_expect(bad < 0, 0)) {
+#pragma unroll 1
+        for (int j = 0; j < R; ++j) {
+            uint32_t x[4];
+            wave_exact<P>(data, pal, j ? start[R - 1] : start[0], j ? end[R - 1] : end[0], n, lane, x);
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                E[0][g] = j == 0 ? x[g] : E[0][g];
+                E[R - 1][g] = j == R - 1 ? x[g] : E[R - 1][g];
+            }
+        }
+    }
+    if (n < 1024) {
+        const int32_t valid = (int32_t)n - 16 * (int32_t)lane;
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            const uint32_t keep = valid >= 4 * g + 4 ? ~0u : keep_bits(~0u, 8 * (valid - 4 * g), 24);
+#pragma unroll
+            for (int j = 0; j < R; ++j) E[j][g] &= keep;
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < R; ++j)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            const uint32_t L = s[j].lit[g];
+            hi[j][g] = (L & 0x80808080u) | ((E[j][g] >> 1) & 0x7F7F7F7Fu);
+            lo[j][g] = (L & 0x7F7F7F7Fu) | ((E[j][g] << 7) & 0x80808080u);
+        }
+}
+
+// The lane's pair words (weights 16l + 2i, + 1) of a decoded block.
+__device__ __forceinline__ void wave_pairs(const uint32_t (&hi)[4], const uint32_t (&lo)[4], uint32_t (&wp)[8]) {
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+        wp[2 * g] = __builtin_amdgcn_perm(hi[g], lo[g], 0x05010400u);
+        wp[2 * g + 1] = __builtin_amdgcn_perm(hi[g], lo[g], 0x07030602u);
+    }
+}
+
+// ---- sums over the lanes
+
+template <int CTRL>
+__device__ __forceinline__ float dpp_move(float v) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true));
+}
+// Lanes 0..31: a summed over lanes l, l + 32; lanes 32..63: b so.
+__device__ __forceinline__ float fold32(float a, float b) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+// The same over rows of 16 lanes: even rows a (l, l + 16), odd rows b.
+__device__ __forceinline__ float fold16(float a, float b) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+// Lanes with `bit` clear: a plus its partner's a; with it set: b so.
+template <int CTRL>
+__device__ __forceinline__ float fold_dpp(float a, float b, bool bit) {
+    const float keep = bit ? b : a, give = bit ? a : b;
+    return keep + dpp_move<CTRL>(give);
+}
+
+// V values (2..16) summed over the 64 lanes: value i in the lanes with
+// lane / (64 / V) == i. The tree is the same for every V: partners at lane
+// distance 32, 16 and 8, the mirror within 8, then 2 and 1.
+template <int V>
+__device__ __forceinline__ float wave_fold(float (&v)[V], uint32_t lane) {
+    constexpr int V1 = V / 2, V2 = V1 > 1 ? V1 / 2 : 1, V3 = V2 > 1 ? V2 / 2 : 1;
+#pragma unroll
+    for (int i = 0; i < V1; ++i) v[i] = fold32(v[i], v[i + V1]);
+#pragma unroll
+    for (int i = 0; i < V2; ++i) v[i] = fold16(v[i], v[V1 > 1 ? i + V2 : i]);
+#pragma unroll
+    for (int i = 0; i < V3; ++i) v[i] = V2 > 1 ? fold_dpp<0x128>(v[i], v[i + V3], lane & 8u) : v[i] + dpp_move<0x128>(v[i]);
+    float s = V3 > 1 ? fold_dpp<0x141>(v[0], v[V3 > 1 ? 1 : 0], lane & 4u) : v[0] + dpp_move<0x141>(v[0]);
+    s += dpp_move<0x4E>(s);
+    return s + dpp_move<0xB1>(s);
+}
+
+// ---- decode + GEMV
+
+struct WaveGroup {
+    const uint32_t* data[kGroupMax];  // the raw weight in kWaveRaw
+    const uint32_t* offsets[kGroupMax];
+    const uint32_t* palette[kGroupMax];
+    const void* bias[kGroupMax];
+    void* out[kGroupMax];
+    uint32_t rows[kGroupMax];
+    uint32_t wg0[kGroupMax + 1];  // tensor i's workgroups: wg0[i] .. wg0[i + 1] - 1
+};
+
+struct WaveShape {
+    uint32_t cols, nb;
+    uint32_t tile;  // T: rows per workgroup, even
+    uint32_t m;     // activation rows (<= the kernel's M; the rest repeat the last one)
+    uint32_t wide;  // 1: x's rows (raw: the weight's too) may be read four bytes at a time
+    int x_dtype, bias_dtype, out_dtype;
+};
+
+struct __attribute__((packed, aligned(4))) Quad4 {
+    uint32_t v[4];
+};
+
+// Waves per workgroup, and the waves per SIMD the registers are cut to: two
+// 8-wave workgroups a CU (128 registers a wave) where the decode and the
+// activations fit that, one 12-wave workgroup (168) where they do not, one
+// 8-wave workgroup (256) for fp32 activations at M = 8 (128 registers of
+// them).
+constexpr bool wave_wide(int P, int M, int XT) {
+    return (P == kWaveBalanced || P == kWaveGulp) && M == (XT == kWaveX32 ? 4 : 8);
+}
+constexpr uint32_t wave_waves(int P, int M, int XT) { return wave_wide(P, M, XT) ? 12u : 8u; }
+constexpr uint32_t wave_occ(int P, int M, int XT) { return wave_wide(P, M, XT) ? 3u : XT == kWaveX32 && M == 8 ? 2u : 4u; }
+constexpr uint32_t kDecodeWaves = 8;
+// static LDS of the wave kernel
+constexpr size_t wave_lds(int P, uint32_t W) { return 8 * ((size_t)W * wave_exchange(P) + WaveTables::entries(P)); }
+static_assert(wave_exchange(kWaveSip) % 2 == 0 && wave_exchange(kWaveBalanced) % 2 == 0 && wave_exchange(kWaveGulp) % 2 == 0,
+              "the exchanges are whole uint2");
+
+template <int P, int M, int XT>
+__global__ __launch_bounds__(wave_waves(P, M, XT) * 64, wave_occ(P, M, XT))
+void k_gemv_wave(const WaveGroup g, const void* __restrict__ x, const WaveShape sh) {
+    constexpr uint32_t W = wave_waves(P, M, XT);
+    constexpr int XR = XT == kWaveX32 ? 16 : 8;  // activation registers per row
+    __shared__ __align__(16) uint2 lds[W * wave_exchange(P) + WaveTables::entries(P)];
+    uint2* tab = lds + W * wave_exchange(P);
+    extern __shared__ __align__(16) uint8_t lds_dyn[];
+    float* red = reinterpret_cast<float*>(lds_dyn);
+
+    const uint32_t wv = wave_id(), lane = lane_id();
+    uint32_t it = 0;
+#pragma unroll
+    for (int i = 1; i < kGroupMax; ++i) it += blockIdx.x >= g.wg0[i];
+    const uint32_t* data = pick(g.data, it);
+    const uint32_t* offsets = pick(g.offsets, it);
+    const uint32_t* palette = pick(g.palette, it);
+    const uint32_t rows = pick(g.rows, it);
+    uint32_t wg0 = g.wg0[0];
+#pragma unroll
+    for (int i = 1; i < kGroupMax; ++i) wg0 = it == (uint32_t)i ? g.wg0[i] : wg0;
+    const uint32_t r0 = (blockIdx.x - wg0) * sh.tile, nrows = min(sh.tile, rows - r0);
+    const uint32_t pairs = (nrows + 1) / 2, units = pairs * sh.nb;
+    const uint32_t u0 = units * wv / W, u1 = units * (wv + 1) / W;
+    const uint32_t first = r0 * sh.nb;  // the tile's first block
+    uint32_t* ex0 = reinterpret_cast<uint32_t*>(lds) + wv * 2 * wave_exchange(P);
+
+    uint32_t xr[M][XR];
+    // (through one buffer resource, a row's start the scalar offset: 128-bit
+    // loads in a whole block; in the last, partial one a dword each, or an
+    // element where the rows are not dword-aligned, and a lane past the row
+    // takes an offset past the resource: it reads 0 and fetches nothing)
+    const auto rx = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(x), 0, 0x7FFFFFFF, 0x00020000);
+    auto load_x = [&](uint32_t cb) {
+        const uint32_t c0 = cb * 1024 + 16 * lane;
+        constexpr uint32_t size = XT == kWaveX32 ? 4 : 2, per = 4 / size;  // elements a register
+        auto at = [&](uint32_t c) { return c < sh.cols ? c * size : 0x80000000u; };
+        if (sh.wide && cb * 1024 + 1024 <= sh.cols) {
+#pragma unroll
+            for (int m = 0; m < M; ++m)
+#pragma unroll
+                for (int i = 0; i < XR / 4; ++i) {
+                    const auto v = __builtin_amdgcn_raw_buffer_load_b128(
+                        rx, c0 * size + 16 * i, min((uint32_t)m, sh.m - 1) * sh.cols * size, 0);
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) xr[m][4 * i + k] = v[k];
+                }
+        } else if (XT == kWaveX32 || sh.wide) {
+#pragma unroll
+            for (uint32_t i = 0; i < XR; ++i) {
+                const uint32_t o = at(c0 + per * i);
+#pragma unroll
+                for (int m = 0; m < M; ++m)
+                    xr[m][i] = __builtin_amdgcn_raw_buffer_load_b32(rx, o, min((uint32_t)m, sh.m - 1) * sh.cols * size, 0);
+            }
+        } else {
+#pragma unroll
+            for (uint32_t i = 0; i < XR; ++i) {
+                const uint32_t o = at(c0 + 2 * i), o1 = at(c0 + 2 * i + 1);
+#pragma unroll
+                for (int m = 0; m < M; ++m) {
+                    const uint32_t row = min((uint32_t)m, sh.m - 1) * sh.cols * size;
+                    xr[m][i] = (uint32_t)(uint16_t)__builtin_amdgcn_raw_buffer_load_b16(rx, o, row, 0) |
+                               (uint32_t)(uint16_t)__builtin_amdgcn_raw_buffer_load_b16(rx, o1, row, 0) << 16;
+                }
+            }
+        }
+    };
+    // the activations waited on here, so that no later use of them waits on
+    // loads issued after
+    auto pin_x = [&]() {
+#pragma unroll
+        for (int m = 0; m < M; ++m)
+#pragma unroll
+            for (int i = 0; i < XR; ++i) asm volatile("" : "+v"(xr[m][i]));
+    };
+
+    // the directory entries of the next 32 units, one block a lane
+    uint32_t o_start = 0, o_end = 0;
+    auto load_directory = [&](uint32_t u) {
+        if constexpr (P != kWaveRaw) {
+            const uint32_t uu = min(u + (lane >> 1), u1 - 1), cb = uu / pairs, pr = uu - cb * pairs;
+            const uint32_t blk = first + min(2 * pr + (lane & 1u), nrows - 1) * sh.nb + cb;
+            o_start = offsets[blk];
+            o_end = offsets[blk + 1];
+        }
+    };
+    auto weights = [&](uint32_t cb) { return min(1024u, sh.cols - cb * 1024); };
+    struct Unit {
+        WaveStage s[2];
+    };
+    auto load_unit = [&](Unit& t, uint32_t k, uint32_t cb, bool live) {
+        if constexpr (P != kWaveRaw) {
+#pragma unroll
+            for (uint32_t j = 0; j < 2; ++j)
+                t.s[j] = wave_load<P>(data, __builtin_amdgcn_readlane(o_start, 2 * k + j),
+                                      __builtin_amdgcn_readlane(o_end, 2 * k + j), weights(cb), live, lane);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto process = [&](const Unit& t, uint32_t k, uint32_t cb, uint32_t pr) {
+        float v[2 * M];
+        uint32_t hi2[2][4], lo2[2][4];
+        if constexpr (P != kWaveRaw) {
+            const uint32_t start[2] = {(uint32_t)__builtin_amdgcn_readlane(o_start, 2 * k),
+                                       (uint32_t)__builtin_amdgcn_readlane(o_start, 2 * k + 1)};
+            const uint32_t end[2] = {(uint32_t)__builtin_amdgcn_readlane(o_end, 2 * k),
+                                     (uint32_t)__builtin_amdgcn_readlane(o_end, 2 * k + 1)};
+            wave_decode<P, 2>(tab, ex0, t.s, data, reinterpret_cast<const uint8_t*>(palette), start, end, weights(cb), lane,
+                              hi2, lo2);
+        }
+#pragma unroll
+        for (uint32_t j = 0; j < 2; ++j) {
+            uint32_t wp[8];
+            const uint32_t(&hi)[4] = hi2[j], (&lo)[4] = lo2[j];
+            if constexpr (P == kWaveRaw) {
+                const uint32_t c0 = cb * 1024 + 16 * lane, n = sh.cols > c0 ? min(16u, sh.cols - c0) : 0u;
+                const uint16_t* w = reinterpret_cast<const uint16_t*>(data) +
+                                    (uint64_t)(r0 + min(2 * pr + j, nrows - 1)) * sh.cols + c0;
+#pragma unroll
+                for (uint32_t i = 0; i < 8; ++i)
+                    wp[i] = (2 * i < n ? (uint32_t)w[2 * i] : 0u) | (2 * i + 1 < n ? (uint32_t)w[2 * i + 1] << 16 : 0u);
+            }
+            if constexpr (XT == kWaveX32) {
+                float w[16];
+#pragma unroll
+                for (int i = 0; i < 16; ++i) {
+                    if constexpr (P == kWaveRaw)
+                        w[i] = __uint_as_float(i & 1 ? wp[i / 2] & 0xFFFF0000u : wp[i / 2] << 16);
+                    else
+                        w[i] = __uint_as_float(__builtin_amdgcn_perm(hi[i / 4], lo[i / 4], ((4u + i % 4) << 24) | ((i % 4) << 16) | 0x0C0Cu));
+                }
+#pragma unroll
+                for (int m = 0; m < M; ++m) {
+                    float a = w[0] * __uint_as_float(xr[m][0]), b = w[1] * __uint_as_float(xr[m][1]);
+#pragma unroll
+                    for (int i = 2; i < 16; i += 2) {
+                        a = fmaf(w[i], __uint_as_float(xr[m][i]), a);
+                        b = fmaf(w[i + 1], __uint_as_float(xr[m][i + 1]), b);
+                    }
+                    v[j * M + m] = a + b;
+                }
+            } else {
+                if constexpr (P != kWaveRaw) wave_pairs(hi, lo, wp);
+#pragma unroll
+                for (int m = 0; m < M; ++m) {
+                    float a = dot2(wp[0], xr[m][0], 0.0f), b = dot2(wp[1], xr[m][1], 0.0f);
+#pragma unroll
+                    for (int i = 2; i < 8; i += 2) {
+                        a = dot2(wp[i], xr[m][i], a);
+                        b = dot2(wp[i + 1], xr[m][i + 1], b);
+                    }
+                    v[j * M + m] = a + b;
+                }
+            }
+        }
+        const float s = wave_fold<2 * M>(v, lane);
+        constexpr uint32_t span = 64 / (2 * M);
+        if (lane % span == 0) {
+            const uint32_t i = lane / span;  // value i: row i / M of the unit, activation row i % M
+            red[((2 * pr + i / M) * sh.nb + cb) * M + i % M] = s;
+        }
+    };
+
+    if (u0 < u1) load_directory(u0);
+    uint32_t cb = u0 / pairs, pr = u0 - cb * pairs;
+    Unit a, b;
+    load_unit(a, 0, cb, u0 < u1);
+    load_x(min(cb, sh.nb - 1));
+    wave_tables<P>(tab, palette, W * 64);
+    __syncthreads();
+    pin_x();
+    // unit k of the run is in flight (in a or b) when its turn comes; its
+    // successor's loads are issued first
+    for (uint32_t u = u0; u < u1;) {
+        const uint32_t n = min(32u, u1 - u);
+        for (uint32_t k = 0; k < n; k += 2) {
+            uint32_t pr1 = pr + 1, cb1 = cb;
+            if (pr1 == pairs) pr1 = 0, ++cb1;
+            load_unit(b, (k + 1) & 31u, min(cb1, sh.nb - 1), k + 1 < n);
+            process(a, k, cb, pr);
+            if (k + 1 < n && cb1 != cb) {
+                load_x(cb1);
+                pin_x();
+            }
+            uint32_t pr2 = pr1 + 1, cb2 = cb1;
+            if (pr2 == pairs) pr2 = 0, ++cb2;
+            load_unit(a, (k + 2) & 31u, min(cb2, sh.nb - 1), k + 2 < n);
+            if (k + 1 < n) process(b, k + 1, cb1, pr1);
+            cb = cb2, pr = pr2;
+            if (k + 2 < n && cb2 != cb1) {
+                load_x(cb2);
+                pin_x();
+            }
+        }
+        u += n;
+        if (u < u1) {  // (n was 32: cb, pr are unit u's)
+            load_directory(u);
+            load_unit(a, 0, cb, true);
+            load_x(cb);
+            pin_x();
+        }
+    }
+    __syncthreads();
+    const void* bias = pick(g.bias, it);
+    void* out = pick(g.out, it);
+    for (uint32_t i = threadIdx.x; i < nrows * sh.m; i += W * 64) {
+        const uint32_t m = i / nrows, t = i - m * nrows;
+        float sum = 0.0f;
+        for (uint32_t c = 0; c < sh.nb; ++c) sum += red[(t * sh.nb + c) * M + m];
+        if (bias) sum += load_elem(bias, sh.bias_dtype, r0 + t);
+        store_elem(out, sh.out_dtype, (uint64_t)m * rows + r0 + t, sum);
+    }
+}
+
+// ---- decode
+
+// Every block to its bf16 bits: a wave takes `run` consecutive blocks (at
+// most 64, whose directory entries its lanes hold), the next one's loads in
+// flight while it decodes and stores one. wide: the output's rows may be
+// written four bytes at a time.
+template <int P>
+__global__ __launch_bounds__(kDecodeWaves * 64, 4) void k_decode_wave(Desc d, uint16_t* __restrict__ out, uint32_t run,
+                                                                     uint32_t wide) {
+    constexpr uint32_t W = kDecodeWaves;
+    __shared__ __align__(16) uint2 lds[W * wave_exchange(P) / 2 + WaveTables::entries(P)];
+    uint2* tab = lds + W * wave_exchange(P) / 2;
+    const uint32_t wv = wave_id(), lane = lane_id(), blocks = d.rows * d.nb;
+    const uint32_t b0 = min(blocks, (blockIdx.x * W + wv) * run), n = min(run, blocks - b0);
+    uint32_t* ex = reinterpret_cast<uint32_t*>(lds) + wv * wave_exchange(P);
+    uint32_t o_start = 0, o_end = 0;
+    if (lane < n) {
+        o_start = d.offsets[b0 + lane];
+        o_end = d.offsets[b0 + lane + 1];
+    }
+    auto weights = [&](uint32_t c) { return min(1024u, d.cols - c * 1024); };
+    auto load = [&](uint32_t k, uint32_t c, bool live) {
+        const WaveStage s = wave_load<P>(d.data, __builtin_amdgcn_readlane(o_start, k & 63u),
+                                         __builtin_amdgcn_readlane(o_end, k & 63u), weights(c), live, lane);
+        __builtin_amdgcn_sched_barrier(0);
+        return s;
+    };
+    auto finish = [&](const WaveStage& s, uint32_t k, uint32_t row, uint32_t c) {
+        uint32_t hi[1][4], lo[1][4], wp[8];
+        const uint32_t w = weights(c);
+        const WaveStage st[1] = {s};
+        const uint32_t start[1] = {(uint32_t)__builtin_amdgcn_readlane(o_start, k)};
+        const uint32_t end[1] = {(uint32_t)__builtin_amdgcn_readlane(o_end, k)};
+        wave_decode<P, 1>(tab, ex, st, d.data, d.table, start, end, w, lane, hi, lo);
+        wave_pairs(hi[0], lo[0], wp);
+        uint16_t* dst = out + (uint64_t)row * d.cols + c * 1024 + 16 * lane;
+        if (wide && 16 * lane + 16 <= w) {
+            reinterpret_cast<Quad4*>(dst)[0] = Quad4{{wp[0], wp[1], wp[2], wp[3]}};
+            reinterpret_cast<Quad4*>(dst)[1] = Quad4{{wp[4], wp[5], wp[6], wp[7]}};
+        } else {
+#pragma unroll
+            for (uint32_t i = 0; i < 16; ++i)
+                if (16 * lane + i < w) dst[i] = (uint16_t)(wp[i / 2] >> (16 * (i & 1)));
+        }
+    };
+    uint32_t row = b0 / d.nb, c = b0 - row * d.nb;
+    WaveStage a = load(0, c, n != 0), b;
+    wave_tables<P>(tab, reinterpret_cast<const uint32_t*>(d.table), W * 64);
+    __syncthreads();
+    for (uint32_t k = 0; k < n; k += 2) {
+        uint32_t row1 = row, c1 = c + 1;
+        if (c1 == d.nb) c1 = 0, ++row1;
+        b = load(k + 1, c1, k + 1 < n);
+        finish(a, k, row, c);
+        row = row1, c = c1 + 1;
+        if (c == d.nb) c = 0, ++row;
+        a = load(k + 2, c, k + 2 < n);
+        if (k + 1 < n) finish(b, k + 1, row1, c1);
+    }
+}

@@ -1,0 +1,109 @@
+"""GPU: the wave kernels (k_gemv_wave, k_decode_wave), which serve 1024-weight
+blocks of every profile where the sip and gulp kernels do not: columns that
+are not whole blocks, the balanced profile, fp32 activations. Against the
+oracle, at the sizes where their split can go wrong: one weight, one row, odd
+row counts (a unit's second row missing), a last block of 1, 4 and 1023
+weights, columns that are not dword-aligned, one block a row, more units than
+one directory read (32) a wave; and at escape densities from none to past
+every limit of the in-register tiers (512 tier-0 and 128 tier-1 escapes, 64
+tail words), which take the reads from memory."""
+
+import zlib
+
+import numpy as np
+import pytest
+
+from oracle import radix_oracle as O
+from tests.helpers import bf16_tensor, escape_heavy_bits, finite_bits, pack_to_dict, u16_of
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [(1, 1025), (3, 1028), (5, 2047), (130, 260), (17, 3079), (1000, 2052), (1030, 9476), (97, 20484)]
+
+
+def _bits(rng, kind, shape):
+    if kind == "tight":
+        return finite_bits(rng, shape)
+    if kind == "spread":
+        return finite_bits(rng, shape, spread=True)
+    return escape_heavy_bits(rng, shape, {"none": 0.0, "dense": 0.35}[kind])
+
+
+@pytest.mark.parametrize("profile", ["sip", "balanced", "gulp"])
+@pytest.mark.parametrize("shape", SHAPES)
+def test_decode_and_gemv_against_the_oracle(cuda, profile, shape):
+    import torch
+
+    from drinkme_amd import radix_ops, swap
+
+    R, C = shape
+    rng = np.random.default_rng(zlib.crc32(repr((profile, shape)).encode()))
+    for kind in ("tight", "spread", "none", "dense"):
+        bits = _bits(rng, kind, shape)
+        p = O.pack(bits, profile, allow_raw=False)
+        rt = swap.to_device_radix(pack_to_dict(p, profile), cuda)
+        print(f"case wave {profile} {shape} {kind}", flush=True)
+        assert np.array_equal(u16_of(radix_ops.decode_bits(rt)), bits), kind
+        xf = rng.standard_normal((8, C)).astype(np.float32)
+        for dtype in (torch.float32, torch.bfloat16):
+            # (rows starting one element into a buffer: the bf16 ones are not dword-aligned)
+            buf = torch.empty(8 * C + 1, dtype=dtype, device=cuda)
+            x = buf[1:].view(8, C)
+            x.copy_(torch.from_numpy(xf))
+            ref, bound = O.gemv_f64(bits, x.float().cpu().numpy())
+            rows = radix_ops.gemv_rows(rt, x, None, torch.float32)
+            err = np.abs(rows.cpu().numpy().astype(np.float64) - ref) / bound
+            assert err.max() <= 1.0, f"{kind} {dtype}: err/bound {err.max():.3g}"
+            # every row the same at any M and alignment, up to the kernels' own order of sums where
+            # bf16 rows of whole blocks run elsewhere (no shape here has whole blocks)
+            for M in (1, 2, 3, 5):
+                assert torch.equal(radix_ops.gemv_rows(rt, x[:M].clone(), None, torch.float32), rows[:M]), f"{kind} M={M}"
+            bias = torch.from_numpy(rng.standard_normal(R).astype(np.float32)).to(cuda)
+            fused = radix_ops.gemv_rows(rt, x[:2], bias, torch.bfloat16)
+            assert torch.equal(fused, (rows[:2] + bias).to(torch.bfloat16)), f"{kind}: fused epilogue"
+
+
+@pytest.mark.parametrize("profile,dtype", [("sip", "float32"), ("balanced", "bfloat16"), ("gulp", "float32")])
+def test_whole_blocks_and_groups(cuda, profile, dtype):
+    """Whole-block columns (their fp32 and balanced route) and a group of
+    three tensors in one launch: each output is its own launch's, bit for
+    bit."""
+    import torch
+
+    from drinkme_amd import radix_ops, swap
+
+    rng = np.random.default_rng(zlib.crc32((profile + dtype).encode()))
+    C = 4096
+    ps, srcs = [], []
+    for R in (1027, 64, 2):
+        bits = finite_bits(rng, (R, C), spread=True)
+        srcs.append(bits)
+        ps.append(swap.to_device_radix(pack_to_dict(O.pack(bits, profile, allow_raw=False), profile), cuda))
+    for M in (1, 4, 7):
+        x = torch.from_numpy(rng.standard_normal((M, C)).astype(np.float32)).to(cuda).to(getattr(torch, dtype))
+        print(f"case wave group {profile} {dtype} M={M}", flush=True)
+        outs = radix_ops.gemv_group(ps, x, None, torch.float32)
+        for p, bits, y in zip(ps, srcs, outs):
+            assert torch.equal(y, radix_ops.gemv_rows(p, x, None, torch.float32))
+            ref, bound = O.gemv_f64(bits, x.float().cpu().numpy())
+            assert np.all(np.abs(y.cpu().numpy().astype(np.float64) - ref) <= bound)
+
+
+def test_a_non_finite_weight_past_the_row_end_is_not_multiplied(cuda):
+    """Palette entry 0 is the exponent of infinities here: the lanes past a
+    row's last column must not bring it (0 x inf) into the sums."""
+    import torch
+
+    from drinkme_amd import radix_ops, swap
+
+    rng = np.random.default_rng(5)
+    bits = finite_bits(rng, (8, 1028))
+    bits[:6, :1024] = 255 << 7  # six rows of infinities, two finite ones
+    x = torch.ones(1, 1028, device=cuda)
+    for profile in ("sip", "balanced", "gulp"):
+        rt = swap.to_device_radix(pack_to_dict(O.pack(bits, profile, allow_raw=False), profile), cuda)
+        assert rt["rx_palette_np"][0] == 255
+        assert np.array_equal(u16_of(radix_ops.decode_bits(rt)), bits)
+        for xx in (x, x.to(torch.bfloat16)):
+            y = radix_ops.gemv_rows(rt, xx, None, torch.float32).cpu().numpy()[0]
+            assert np.all(np.isinf(y[:6])) and np.all(np.isfinite(y[6:])), profile
