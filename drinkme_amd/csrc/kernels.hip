@@ -2340,10 +2340,10 @@ int launch_wave(int p, const dmx_radix_tensor* const* ts, uint32_t n, const void
     sh.bias_dtype = bias_dtype;
     sh.out_dtype = out_dtype;
     sh.wide = xt == kWaveX32 || (sh.cols % 2 == 0 && reinterpret_cast<uintptr_t>(x) % 4 == 0);
-    uint64_t rows = 0;
-    for (uint32_t i = 0; i < n; ++i) rows += ts[i]->rows;
+    uint32_t rows[kGroupMax];
+    for (uint32_t i = 0; i < n; ++i) rows[i] = ts[i]->rows;
     const uint32_t M = 1u << mi, W = wave_waves(p, (int)M, xt);
-    sh.tile = wave_tile(rows, sh.nb, M, (uint32_t)cu_count() * wave_occ(p, (int)M, xt) * 4u / W, wave_lds(p, W));
+    sh.tile = wave_tile(rows, n, sh.nb, M, W, (uint32_t)cu_count() * wave_occ(p, (int)M, xt) * 4u / W, wave_lds(p, W));
     if (sh.tile == 0) return 2;
     WaveGroup g;
     uint64_t wgs = 0;

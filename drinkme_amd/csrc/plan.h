@@ -566,17 +566,40 @@ inline bool plan_gulp(SipShape& sh, const uint32_t* row0, uint32_t n, uint32_t m
     return true;
 }
 
-// The wave kernel's rows per workgroup T: even, enough that the group's rows
-// make about `slots` workgroups, the ones the chip holds at once, and no
-// more than keep a tile's sums (one float per row, column block and
-// activation row) to 16 KB, and with the kernel's static LDS `fixed` to 64
-// KB, so two workgroups fit a CU. 0: not even two rows fit.
+// The wave kernel's rows per workgroup T (even) for n tensors of rows[i]
+// rows and nb column blocks: the T that takes the fewest unit times, a
+// workgroup's being its waves' longest run of units and kWaveSetup of them
+// for its start and end, and workgroups beyond the `slots` that the chip
+// holds at once running as later rounds. (Two workgroups too many double a
+// short launch: balanced q/k/v of 6144 x 4096 at T = 12, 514 workgroups for
+// 512 slots, took 14.8 us, 4096 x 4096 alone 9.6.) Tried: the even tiles
+// that fill one to four rounds, and the next two. A tile's sums (one float
+// per row, column block and activation row) stay within 16 KB, and with the
+// kernel's static LDS `fixed` within 64 KB. 0: not even two rows fit.
 constexpr size_t kWaveSums = 16 * 1024;
-inline uint32_t wave_tile(uint64_t rows, uint32_t nb, uint32_t M, uint32_t slots, size_t fixed) {
+constexpr uint32_t kWaveSetup = 3;
+inline uint32_t wave_tile(const uint32_t* rows, uint32_t n, uint32_t nb, uint32_t M, uint32_t W, uint32_t slots,
+                          size_t fixed) {
+    uint64_t total = 0;
+    for (uint32_t i = 0; i < n; ++i) total += rows[i];
     const uint64_t row_bytes = (uint64_t)nb * M * 4;
     const uint64_t most = std::min(kWaveSums, 64 * 1024 - fixed) / row_bytes & ~1ull;
-    const uint64_t even = ((rows + slots - 1) / slots + 1) & ~1ull;
-    return (uint32_t)std::min(most, std::max<uint64_t>(even, 2));
+    uint64_t best = 0, best_cost = ~0ull;
+    for (uint32_t r = 1; r <= 4; ++r) {
+        const uint64_t even = ((total + (uint64_t)slots * r - 1) / ((uint64_t)slots * r) + 1) & ~1ull;
+        for (uint64_t t = std::max<uint64_t>(even, 2); t <= even + 4; t += 2) {
+            const uint64_t tile = std::min(t, most);
+            if (tile == 0) return 0;
+            uint64_t wgs = 0;
+            for (uint32_t i = 0; i < n; ++i) wgs += (rows[i] + tile - 1) / tile;
+            const uint64_t cost = ((wgs + slots - 1) / slots) * ((tile / 2 * nb + W - 1) / W + kWaveSetup);
+            if (cost < best_cost) {
+                best_cost = cost;
+                best = tile;
+            }
+        }
+    }
+    return (uint32_t)best;
 }
 
 }  // namespace dmx

@@ -15,13 +15,14 @@
 // end. Every sum is a function of the row and the activation alone: the
 // same for any M, T and W.
 //
-// What bounds it: VALU issue (80% busy between a launch's start and end: 91
-// VALU instructions a sip block, 106 a balanced one at M = 1 bf16, 16 M + 16
-// more for the fp32 products), then the 3 us of a launch before and after
-// its blocks. Measured, one launch, against k_gemv_generic, which scans
-// over a workgroup with two barriers a tier: sip 2 x 9472 x 3584 (ragged)
-// 24.5 us for 284, sip 3584 x 9472 15.8 for 149; gulp fp32 M = 2 q/k/v of
-// 10240 x 5120 31.4 for 326; balanced q/k/v of 6144 x 4096 16.0 for 145.
+// What bounds it: for launches of a few units a wave, the 6 us before and
+// after them (the directory's round trip, the first payload, the tables);
+// for longer ones the payload's stream and the VALU (80 instructions a sip
+// block at M = 1 bf16, 95 to 105 with more tiers, 16 M + 16 more for fp32
+// products). Measured, one launch, against k_gemv_generic, which scans over
+// a workgroup with two barriers a tier: sip 2 x 9472 x 3584 (ragged) 21.2 us
+// for 284, sip 3584 x 9472 14.3 for 149; gulp fp32 M = 2 q/k/v of 10240 x
+// 5120 23.8 for 326; balanced q/k/v of 6144 x 4096 12.8 for 145.
 //
 // The decode works on bytes. A table entry holds four exponent bytes and a
 // v_perm selector over (four consecutive bytes of the next tier's
@@ -79,22 +80,33 @@ struct WaveTables {
     static constexpr uint32_t tier(int P, uint32_t j) { return j == 0 ? 0u : j == 1 ? 256u : 512u; }
 };
 
-// A wave's LDS exchange, in words, per row of a unit: the tail words and one
-// more, the tier-1 exponent bytes (512 and a window's overhang) and the
-// tier-2 ones (128 and the overhang).
-constexpr uint32_t kExTail = 0, kExT1 = 66, kExT2 = kExT1 + 130;
+// A wave's LDS exchange, in words, per row of a unit: the tail words rotated
+// (read as terminal bytes) and, past one tier, as they are (read as codes),
+// each with one word more; the tier-1 exponent bytes (512 and a window's
+// overhang) and the tier-2 ones (128 and the overhang).
+constexpr uint32_t kExTerm = 0, kExTail = 66, kExT1 = 132, kExT2 = kExT1 + 130;
 constexpr uint32_t wave_exchange(int P) {
-    return P == kWaveSip ? kExT1 : P == kWaveBalanced ? kExT2 : P == kWaveGulp ? kExT2 + 34 : 0u;
+    return P == kWaveSip ? kExTail : P == kWaveBalanced ? kExT2 : P == kWaveGulp ? kExT2 + 34 : 0u;
 }
 
-// Four bytes at byte address `at` of LDS words: the two words holding them
-// and a funnel shift. (One unaligned ds_read_b32 instead stalls the LDS for
-// about 60 cycles a wave: the 9472 x 3584 gate/up launch took 45.6 us with
-// it, 28.8 us without.)
-__device__ __forceinline__ uint32_t lds_bytes(const uint32_t* words, uint32_t at) {
-    const uint32_t* p = reinterpret_cast<const uint32_t*>(reinterpret_cast<const uint8_t*>(words) + (at & ~3u));
-    return __builtin_amdgcn_alignbyte(p[1], p[0], at);
+// Exponent bytes are kept rotated right by one: a byte's low seven bits are
+// the bf16 high byte's and its top bit the low byte's, so merging them with
+// the literals (sign and mantissa) takes one v_bfi a half.
+__device__ __forceinline__ uint32_t rotate_bytes(uint32_t v) {
+    return ((v >> 1) & 0x7F7F7F7Fu) | ((v << 7) & 0x80808080u);
 }
+
+// Two words of LDS from byte address `at` on, `at` rounded down to a word,
+// and the four bytes from `at` in them. (One unaligned ds_read_b32 instead
+// stalls the LDS for about 60 cycles a wave: the 9472 x 3584 gate/up launch
+// took 45.6 us with it, 28.8 us without.)
+typedef const __attribute__((address_space(3))) uint32_t* lds_words;
+__device__ __forceinline__ uint32_t lds_address(const void* p) { return (uint32_t)(uintptr_t)(lds_ptr)p; }
+__device__ __forceinline__ uint2 lds_window(uint32_t at) {
+    const lds_words p = (lds_words)(uintptr_t)(at & ~3u);
+    return make_uint2(p[0], p[1]);
+}
+__device__ __forceinline__ uint32_t window_bytes(uint2 w, uint32_t at) { return __builtin_amdgcn_alignbyte(w.y, w.x, at); }
 
 // Entry of four codes c[k] < 2^w, exponents from the run `pal` of the padded
 // tables (the escape code reads its zero pad byte).
@@ -106,7 +118,7 @@ __device__ __forceinline__ uint2 wave_entry(uint32_t i, const uint32_t (&pal)[4]
         const uint32_t c = (i >> (w * k)) & ((1u << w) - 1u);
         uint32_t b = __builtin_amdgcn_perm(pal[1], pal[0], c & 7u);
         if (w == 4) b = c & 8u ? __builtin_amdgcn_perm(pal[3], pal[2], c & 7u) : b;
-        e |= (b & 0xFFu) << (8 * k);
+        e |= (b & 0xFFu) << (8 * k);  // (rotated bytes, as pal's are)
         if (c == (1u << w) - 1u) sel ^= (k ^ r++) << (8 * k);
     }
     return make_uint2(e, sel);
@@ -132,15 +144,16 @@ __device__ __forceinline__ void wave_table3(uint2* tab, uint32_t p0, uint32_t p1
 // Builds the tables of profile P (all of the workgroup's threads).
 template <int P>
 __device__ __forceinline__ void wave_tables(uint2* tab, const uint32_t* palette, uint32_t threads) {
-    const const_u32_ptr p = (const_u32_ptr)palette;
+    const const_u32_ptr pw = (const_u32_ptr)palette;
+    auto p = [&](int i) { return rotate_bytes(pw[i]); };
     if constexpr (P == kWaveSip) {
-        wave_table3(tab, p[0], p[1], threads);
+        wave_table3(tab, p(0), p(1), threads);
     } else if constexpr (P == kWaveBalanced) {
-        const uint32_t pal0[4] = {p[0], 0, 0, 0};
+        const uint32_t pal0[4] = {p(0), 0, 0, 0};
         for (uint32_t i = threadIdx.x; i < 256; i += threads) tab[i] = wave_entry<2, 4>(i, pal0);
-        wave_table3(tab + 256, p[1], p[2], threads);
+        wave_table3(tab + 256, p(1), p(2), threads);
     } else if constexpr (P == kWaveGulp) {
-        const uint32_t pal0[4] = {p[0], 0, 0, 0}, pal1[4] = {p[1], 0, 0, 0}, pal2[4] = {p[2], p[3], p[4], p[5]};
+        const uint32_t pal0[4] = {p(0), 0, 0, 0}, pal1[4] = {p(1), 0, 0, 0}, pal2[4] = {p(2), p(3), p(4), p(5)};
         for (uint32_t i = threadIdx.x; i < 768; i += threads)
             tab[i] = i < 256 ? wave_entry<2, 4>(i, pal0) : i < 512 ? wave_entry<2, 4>(i - 256, pal1)
                                                                   : wave_entry<4, 2>(i - 512, pal2);
@@ -155,9 +168,15 @@ struct WaveStage {
     uint32_t tail;
 };
 
-__device__ __forceinline__ uint32_t block_fixed(int P, uint32_t n) { return words_for(n, 8) + words_for(n, wave_width(P, 0)); }
+// A block's size: n weights, lit words of literals, fixed words with tier 0.
+struct BlockSize {
+    uint32_t n, lit, fixed;
+};
+__device__ __forceinline__ BlockSize block_size(int P, uint32_t n) {
+    return {n, words_for(n, 8), words_for(n, 8) + words_for(n, wave_width(P, 0))};
+}
 
-// Loads block [start, end) of n weights, non-temporal, through a buffer
+// Loads the block of len words at `start`, non-temporal, through a buffer
 // resource that ends four words past the block (or its fixed streams, where
 // the block is cut shorter than those): no wide load of a lane straddles the
 // end, and those words are the next block's or the pad's. The tail's lanes
@@ -165,27 +184,25 @@ __device__ __forceinline__ uint32_t block_fixed(int P, uint32_t n) { return word
 // nothing. live = false: nothing is fetched. The loads are unconditional, so
 // the compiler's waits for one stage leave the next one's loads in flight.
 template <int P>
-__device__ __forceinline__ WaveStage wave_load(const uint32_t* data, uint32_t start, uint32_t end, uint32_t n, bool live,
-                                               uint32_t lane) {
-    const int32_t len = (int32_t)(end - start);
-    const uint32_t lw = words_for(n, 8), fixed = block_fixed(P, n);
-    const uint32_t reach = 4u * ((uint32_t)max(len, (int32_t)fixed) + 4u);
+__device__ __forceinline__ WaveStage wave_load(const uint32_t* data, uint32_t start, int32_t len, const BlockSize& z,
+                                               bool live, uint32_t lane) {
+    const uint32_t reach = 4u * ((uint32_t)max(len, (int32_t)z.fixed) + 4u);
     const auto r = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint32_t*>(data + start), 0, live ? reach : 0u, 0x00020000);
     constexpr int nt = 2;
     WaveStage s;
     s.lit = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, 16 * lane, 0, nt));
     if constexpr (P == kWaveSip) {
-        s.t0 = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(r, 4 * (lw + ((3 * lane) >> 1)), 0, nt));
+        s.t0 = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(r, 4 * (z.lit + ((3 * lane) >> 1)), 0, nt));
     } else {
-        s.t0.x = __builtin_amdgcn_raw_buffer_load_b32(r, 4 * (lw + lane), 0, nt);
+        s.t0.x = __builtin_amdgcn_raw_buffer_load_b32(r, 4 * (z.lit + lane), 0, nt);
         s.t0.y = 0;
     }
     s.tail = __builtin_amdgcn_raw_buffer_load_b32(
-        r, (int32_t)lane < len - (int32_t)fixed ? 4 * (fixed + lane) : 0x80000000u, 0, nt);
+        r, (int32_t)lane < len - (int32_t)z.fixed ? 4 * (z.fixed + lane) : 0x80000000u, 0, nt);
     return s;
 }
 
-// The lane's 16 exponent bytes with every field read from memory, as
+// The lane's 16 exponent bytes (rotated) with every field read from memory, as
 // decode_block reads them (any escape counts, streams of any length).
 template <int P>
 __device__ void wave_exact(const uint32_t* data, const uint8_t* pal, uint32_t start, uint32_t end, uint32_t n,
@@ -223,10 +240,10 @@ __device__ void wave_exact(const uint32_t* data, const uint8_t* pal, uint32_t st
         for (int i = 0; i < 16; ++i)
             if ((active >> i) & 1u) place(i, field(data + pos, r++, 8));
     }
-    E[0] = (uint32_t)elo;
-    E[1] = (uint32_t)(elo >> 32);
-    E[2] = (uint32_t)ehi;
-    E[3] = (uint32_t)(ehi >> 32);
+    E[0] = rotate_bytes((uint32_t)elo);
+    E[1] = rotate_bytes((uint32_t)(elo >> 32));
+    E[2] = rotate_bytes((uint32_t)ehi);
+    E[3] = rotate_bytes((uint32_t)(ehi >> 32));
 }
 
 // The first `bits` (clamped to 0 .. most < 32) bits of codes: those past the
@@ -240,34 +257,35 @@ __device__ __forceinline__ uint32_t add_escapes(uint2 e, uint32_t n) {
     return (uint32_t)__builtin_popcount(e.y & 0x04040404u) + n;
 }
 
-// Completes an entry from the next tier's exponent bytes (at byte `at` of
-// `bytes`, the group's first escape).
-__device__ __forceinline__ uint32_t complete(uint2 e, const uint32_t* bytes, uint32_t at) {
-    return __builtin_amdgcn_perm(lds_bytes(bytes, at), e.x, e.y);
-}
+// Completes an entry from the next tier's four exponent bytes.
+__device__ __forceinline__ uint32_t complete(uint2 e, uint32_t next) { return __builtin_amdgcn_perm(next, e.x, e.y); }
 
-// Decodes R blocks of n weights (R = 2: a unit's rows; 1) from their loaded
+// Decodes R blocks of size z (R = 2: a unit's rows; 1) from their loaded
 // stages: hi[j][g], lo[j][g] = the high and low bytes of the bf16 bits of the
-// lane's weights 4g .. 4g + 3 of block j (weight k in byte k). Weights past n
-// get exponent 0 (a zero or denormal, finite: their activations are 0). ex:
-// the wave's exchange, R x wave_exchange(P) words, in front of the tables, so
-// that a block outside the limits, whose window addresses reach at most 1 KB
-// too far, still reads inside the LDS array.
+// lane's weights 4g .. 4g + 3 of block j (weight k in byte k). Weights past
+// the block get exponent 0 (a zero or denormal, finite: their activations
+// are 0). ex: the wave's exchange, R x wave_exchange(P) words, in front of
+// the tables, so that a block outside the limits, whose window addresses
+// reach at most 1 KB too far, still reads inside the LDS array. The
+// sched_barriers keep a level's LDS reads together: left to itself the
+// compiler waits for each before it issues the next.
 template <int P, int R>
 __device__ __forceinline__ void wave_decode(const uint2* tab, uint32_t* ex, const WaveStage (&s)[R], const uint32_t* data,
-                                            const uint8_t* pal, const uint32_t (&start)[R], const uint32_t (&end)[R],
-                                            uint32_t n, uint32_t lane, uint32_t (&hi)[R][4], uint32_t (&lo)[R][4]) {
+                                            const uint8_t* pal, const uint32_t (&start)[R], const int32_t (&len)[R],
+                                            const BlockSize& z, uint32_t lane, uint32_t (&hi)[R][4],
+                                            uint32_t (&lo)[R][4]) {
     constexpr uint32_t stride = wave_exchange(P);
-    const uint32_t fixed = block_fixed(P, n);
+    const uint32_t ex_at = lds_address(ex);
     uint2 e[R][4];
     uint32_t c[R][4];  // escapes of groups 0 .. g
     int32_t tail[R], bad = 0;  // (bad: negative once a limit is passed; every quantity is far below 2^31)
     uint32_t T[R][2];
 #pragma unroll
     for (int j = 0; j < R; ++j) {
-        tail[j] = (int32_t)(end[j] - start[j] - fixed);
+        tail[j] = len[j] - (int32_t)z.fixed;
         bad |= 64 - tail[j];
-        ex[j * stride + kExTail + lane] = s[j].tail;
+        ex[j * stride + kExTerm + lane] = rotate_bytes(s[j].tail);
+        if constexpr (P != kWaveSip) ex[j * stride + kExTail + lane] = s[j].tail;
         if constexpr (P == kWaveSip) {
             const uint64_t v = ((uint64_t)s[j].t0.y << 32 | s[j].t0.x) >> ((lane & 1) * 16);
             T[j][0] = (uint32_t)v;
@@ -276,8 +294,8 @@ __device__ __forceinline__ void wave_decode(const uint2* tab, uint32_t* ex, cons
             T[j][0] = s[j].t0.x;
         }
     }
-    if (n < 1024) {
-        const int32_t bits = ((int32_t)n - 16 * (int32_t)lane) * (int32_t)wave_width(P, 0);
+    if (z.n < 1024) {
+        const int32_t bits = ((int32_t)z.n - 16 * (int32_t)lane) * (int32_t)wave_width(P, 0);
 #pragma unroll
         for (int j = 0; j < R; ++j) {
             T[j][0] = bits >= 32 ? T[j][0] : keep_bits(T[j][0], bits, 31);
@@ -296,6 +314,7 @@ __device__ __forceinline__ void wave_decode(const uint2* tab, uint32_t* ex, cons
             for (int g = 0; g < 4; ++g) e[j][g] = tab[(T[j][0] >> (8 * g)) & 0xFFu];
         }
     }
+    __builtin_amdgcn_sched_barrier(0);
     // counts of both rows through one scan, row j in bits 16j .. 16j + 15
     uint32_t q[R], n1[R];
     auto scan = [&](const uint32_t (&cnt)[R], uint32_t (&first)[R], uint32_t (&total)[R]) {
@@ -317,7 +336,7 @@ __device__ __forceinline__ void wave_decode(const uint2* tab, uint32_t* ex, cons
         cnt[j] = c[j][3];
     }
     scan(cnt, q, n1);
-    uint32_t bytes = kExTail;  // where tier 0's escapes lie, in words of the exchange
+    uint32_t below = kExTerm;  // where tier 0's escapes lie, in words of the exchange
     if constexpr (P == kWaveSip) {
 #pragma unroll
         for (int j = 0; j < R; ++j) bad |= 4 * tail[j] - (int32_t)n1[j];
@@ -326,20 +345,42 @@ __device__ __forceinline__ void wave_decode(const uint2* tab, uint32_t* ex, cons
         constexpr uint32_t w = wave_width(P, 1);
         uint32_t w1[R], g0[R], q1[R], n2[R];
         uint2 a[R][2];
+        uint2 win[R][2];
+        // the two groups' windows in the exponent bytes at byte `at` of the
+        // exchange, and the groups completed from them
+        uint32_t p1[R];
+        auto windows = [&](int j, uint32_t at) {
+            p1[j] = q1[j] + at;
+            win[j][0] = lds_window(p1[j]);
+            win[j][1] = lds_window(p1[j] + g0[j]);
+        };
+        auto finish = [&]() {
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int j = 0; j < R; ++j) {
+                a[j][0].x = complete(a[j][0], window_bytes(win[j][0], p1[j]));
+                a[j][1].x = complete(a[j][1], window_bytes(win[j][1], p1[j] + g0[j]));
+            }
+        };
 #pragma unroll
         for (int j = 0; j < R; ++j) {
-            const uint32_t* t = ex + j * stride + kExTail;
+            const uint32_t t = ex_at + 4 * (j * stride + kExTail);
             w1[j] = words_for(n1[j], w);
             const int32_t bits = (int32_t)(w * n1[j]) - (int32_t)(8 * w * lane);
             if constexpr (P == kWaveBalanced) {
-                const uint32_t code = keep_bits(lds_bytes(t, 3 * lane), bits, 24);
+                const uint32_t code = keep_bits(window_bytes(lds_window(t + 3 * lane), 3 * lane), bits, 24);
                 a[j][0] = tab[256 + (code & 0xFFFu)];
                 a[j][1] = tab[256 + (code >> 12)];
             } else {
-                const uint32_t code = keep_bits(reinterpret_cast<const uint16_t*>(t)[lane], bits, 16);
+                const uint32_t code =
+                    keep_bits(reinterpret_cast<const uint16_t*>(ex + j * stride + kExTail)[lane], bits, 16);
                 a[j][0] = tab[256 + (code & 0xFFu)];
                 a[j][1] = tab[256 + (code >> 8)];
             }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int j = 0; j < R; ++j) {
             g0[j] = add_escapes(a[j][0], 0);
             cnt[j] = add_escapes(a[j][1], g0[j]);
         }
@@ -349,9 +390,7 @@ __device__ __forceinline__ void wave_decode(const uint2* tab, uint32_t* ex, cons
             for (int j = 0; j < R; ++j) {
                 const int32_t left = tail[j] - (int32_t)w1[j];  // terminal words
                 bad |= (512 - (int32_t)n1[j]) | left | (4 * left - (int32_t)n2[j]);
-                const uint32_t* t = ex + j * stride + kExTail + (w1[j] & 63u);
-                a[j][0].x = complete(a[j][0], t, q1[j]);
-                a[j][1].x = complete(a[j][1], t, q1[j] + g0[j]);
+                windows(j, ex_at + 4 * (j * stride + kExTerm + (w1[j] & 63u)));
             }
         } else {
             // lane l: the block's tier-2 codes 2l, 2l + 1
@@ -362,47 +401,57 @@ __device__ __forceinline__ void wave_decode(const uint2* tab, uint32_t* ex, cons
                 w2[j] = words_for(n2[j], 4);
                 const uint32_t code = reinterpret_cast<const uint8_t*>(ex + j * stride + kExTail + (w1[j] & 63u))[lane];
                 b[j] = tab[512 + keep_bits(code, (int32_t)(4 * n2[j]) - (int32_t)(8 * lane), 8)];
-                cnt[j] = add_escapes(b[j], 0);
                 bad |= (512 - (int32_t)n1[j]) | (128 - (int32_t)n2[j]) | (tail[j] - (int32_t)(w1[j] + w2[j]));
             }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int j = 0; j < R; ++j) cnt[j] = add_escapes(b[j], 0);
             if (__builtin_amdgcn_ballot_w64((cnt[0] | cnt[R - 1]) != 0) != 0) {
                 uint32_t q2[R], n3[R];
                 scan(cnt, q2, n3);
 #pragma unroll
                 for (int j = 0; j < R; ++j) {
                     bad |= 4 * (tail[j] - (int32_t)(w1[j] + w2[j])) - (int32_t)n3[j];
-                    b[j].x = complete(b[j], ex + j * stride + kExTail + ((w1[j] + w2[j]) & 63u), q2[j]);
+                    const uint32_t at = ex_at + 4 * (j * stride + kExTerm + ((w1[j] + w2[j]) & 63u)) + q2[j];
+                    b[j].x = complete(b[j], window_bytes(lds_window(at), at));
                 }
             }
 #pragma unroll
             for (int j = 0; j < R; ++j) reinterpret_cast<uint16_t*>(ex + j * stride + kExT2)[lane] = (uint16_t)b[j].x;
             __builtin_amdgcn_wave_barrier();
 #pragma unroll
-            for (int j = 0; j < R; ++j) {
-                a[j][0].x = complete(a[j][0], ex + j * stride + kExT2, q1[j]);
-                a[j][1].x = complete(a[j][1], ex + j * stride + kExT2, q1[j] + g0[j]);
-            }
+            for (int j = 0; j < R; ++j) windows(j, ex_at + 4 * (j * stride + kExT2));
         }
+        finish();
 #pragma unroll
         for (int j = 0; j < R; ++j)
             *reinterpret_cast<uint2*>(ex + j * stride + kExT1 + 2 * lane) = make_uint2(a[j][0].x, a[j][1].x);
         __builtin_amdgcn_wave_barrier();
-        bytes = kExT1;
+        below = kExT1;
     }
+    uint2 win[R][4];
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+        q[j] += ex_at + 4 * (j * stride + below);
+        win[j][0] = lds_window(q[j]);
+#pragma unroll
+        for (int g = 1; g < 4; ++g) win[j][g] = lds_window(c[j][g - 1] += q[j]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
     uint32_t E[R][4];
 #pragma unroll
     for (int j = 0; j < R; ++j) {
-        const uint32_t* t = ex + j * stride + bytes;
-        E[j][0] = complete(e[j][0], t, q[j]);
+        E[j][0] = complete(e[j][0], window_bytes(win[j][0], q[j]));
 #pragma unroll
-        for (int g = 1; g < 4; ++g) E[j][g] = complete(e[j][g], t, q[j] + c[j][g - 1]);
+        for (int g = 1; g < 4; ++g) E[j][g] = complete(e[j][g], window_bytes(win[j][g], c[j][g - 1]));
     }
     __builtin_amdgcn_wave_barrier();
     if (__builtin_expect(bad < 0, 0)) {
 #pragma unroll 1
         for (int j = 0; j < R; ++j) {
             uint32_t x[4];
-            wave_exact<P>(data, pal, j ? start[R - 1] : start[0], j ? end[R - 1] : end[0], n, lane, x);
+            const uint32_t at = j ? start[R - 1] : start[0];
+            wave_exact<P>(data, pal, at, at + (uint32_t)(j ? len[R - 1] : len[0]), z.n, lane, x);
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
                 E[0][g] = j == 0 ? x[g] : E[0][g];
@@ -410,8 +459,8 @@ __device__ __forceinline__ void wave_decode(const uint2* tab, uint32_t* ex, cons
             }
         }
     }
-    if (n < 1024) {
-        const int32_t valid = (int32_t)n - 16 * (int32_t)lane;
+    if (z.n < 1024) {
+        const int32_t valid = (int32_t)z.n - 16 * (int32_t)lane;
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
             const uint32_t keep = valid >= 4 * g + 4 ? ~0u : keep_bits(~0u, 8 * (valid - 4 * g), 24);
@@ -424,8 +473,8 @@ __device__ __forceinline__ void wave_decode(const uint2* tab, uint32_t* ex, cons
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
             const uint32_t L = s[j].lit[g];
-            hi[j][g] = (L & 0x80808080u) | ((E[j][g] >> 1) & 0x7F7F7F7Fu);
-            lo[j][g] = (L & 0x7F7F7F7Fu) | ((E[j][g] << 7) & 0x80808080u);
+            hi[j][g] = (L & 0x80808080u) | (E[j][g] & 0x7F7F7F7Fu);
+            lo[j][g] = (L & 0x7F7F7F7Fu) | (E[j][g] & 0x80808080u);
         }
 }
 
@@ -508,10 +557,12 @@ struct __attribute__((packed, aligned(4))) Quad4 {
 // 8-wave workgroup (256) for fp32 activations at M = 8 (128 registers of
 // them).
 constexpr bool wave_wide(int P, int M, int XT) {
-    return (P == kWaveBalanced || P == kWaveGulp) && M == (XT == kWaveX32 ? 4 : 8);
+    return P != kWaveRaw && M == (XT == kWaveX32 ? 4 : 8);
 }
 constexpr uint32_t wave_waves(int P, int M, int XT) { return wave_wide(P, M, XT) ? 12u : 8u; }
-constexpr uint32_t wave_occ(int P, int M, int XT) { return wave_wide(P, M, XT) ? 3u : XT == kWaveX32 && M == 8 ? 2u : 4u; }
+constexpr uint32_t wave_occ(int P, int M, int XT) {
+    return wave_wide(P, M, XT) ? 3u : XT == kWaveX32 && M == 8 ? 2u : 4u;
+}
 constexpr uint32_t kDecodeWaves = 8;
 // static LDS of the wave kernel
 constexpr size_t wave_lds(int P, uint32_t W) { return 8 * ((size_t)W * wave_exchange(P) + WaveTables::entries(P)); }
@@ -605,30 +656,39 @@ void k_gemv_wave(const WaveGroup g, const void* __restrict__ x, const WaveShape 
             o_end = offsets[blk + 1];
         }
     };
-    auto weights = [&](uint32_t cb) { return min(1024u, sh.cols - cb * 1024); };
+    constexpr int SP = P == kWaveRaw ? kWaveSip : P;  // (the raw weight has no streams: sizes unused)
+    const BlockSize whole = block_size(SP, 1024), last = block_size(SP, sh.cols - (sh.nb - 1) * 1024);
+    auto size_of = [&](uint32_t cb) {
+        const bool l = cb + 1 == sh.nb;
+        return BlockSize{l ? last.n : whole.n, l ? last.lit : whole.lit, l ? last.fixed : whole.fixed};
+    };
     struct Unit {
         WaveStage s[2];
+        uint32_t start[2];
+        int32_t len[2];
     };
     auto load_unit = [&](Unit& t, uint32_t k, uint32_t cb, bool live) {
         if constexpr (P != kWaveRaw) {
+            const BlockSize z = size_of(cb);
 #pragma unroll
-            for (uint32_t j = 0; j < 2; ++j)
-                t.s[j] = wave_load<P>(data, __builtin_amdgcn_readlane(o_start, 2 * k + j),
-                                      __builtin_amdgcn_readlane(o_end, 2 * k + j), weights(cb), live, lane);
+            for (uint32_t j = 0; j < 2; ++j) {
+                t.start[j] = __builtin_amdgcn_readlane(o_start, 2 * k + j);
+                t.len[j] = (int32_t)(__builtin_amdgcn_readlane(o_end, 2 * k + j) - t.start[j]);
+                t.s[j] = wave_load<P>(data, t.start[j], t.len[j], z, live, lane);
+            }
         }
         __builtin_amdgcn_sched_barrier(0);
     };
-    auto process = [&](const Unit& t, uint32_t k, uint32_t cb, uint32_t pr) {
+    // where the lane's folded sum goes: value i = lane / span is row i / M of
+    // the unit, activation row i % M
+    constexpr uint32_t span = 64 / (2 * M);
+    float* const red_lane = red + (lane / span / M * sh.nb * M + lane / span % M);
+    auto process = [&](const Unit& t, uint32_t cb, uint32_t pr) {
         float v[2 * M];
         uint32_t hi2[2][4], lo2[2][4];
-        if constexpr (P != kWaveRaw) {
-            const uint32_t start[2] = {(uint32_t)__builtin_amdgcn_readlane(o_start, 2 * k),
-                                       (uint32_t)__builtin_amdgcn_readlane(o_start, 2 * k + 1)};
-            const uint32_t end[2] = {(uint32_t)__builtin_amdgcn_readlane(o_end, 2 * k),
-                                     (uint32_t)__builtin_amdgcn_readlane(o_end, 2 * k + 1)};
-            wave_decode<P, 2>(tab, ex0, t.s, data, reinterpret_cast<const uint8_t*>(palette), start, end, weights(cb), lane,
-                              hi2, lo2);
-        }
+        if constexpr (P != kWaveRaw)
+            wave_decode<P, 2>(tab, ex0, t.s, data, reinterpret_cast<const uint8_t*>(palette), t.start, t.len, size_of(cb),
+                              lane, hi2, lo2);
 #pragma unroll
         for (uint32_t j = 0; j < 2; ++j) {
             uint32_t wp[8];
@@ -675,11 +735,7 @@ void k_gemv_wave(const WaveGroup g, const void* __restrict__ x, const WaveShape 
             }
         }
         const float s = wave_fold<2 * M>(v, lane);
-        constexpr uint32_t span = 64 / (2 * M);
-        if (lane % span == 0) {
-            const uint32_t i = lane / span;  // value i: row i / M of the unit, activation row i % M
-            red[((2 * pr + i / M) * sh.nb + cb) * M + i % M] = s;
-        }
+        if (lane % span == 0) red_lane[(2 * pr * sh.nb + cb) * M] = s;
     };
 
     if (u0 < u1) load_directory(u0);
@@ -698,7 +754,7 @@ void k_gemv_wave(const WaveGroup g, const void* __restrict__ x, const WaveShape 
             uint32_t pr1 = pr + 1, cb1 = cb;
             if (pr1 == pairs) pr1 = 0, ++cb1;
             load_unit(b, (k + 1) & 31u, min(cb1, sh.nb - 1), k + 1 < n);
-            process(a, k, cb, pr);
+            process(a, cb, pr);
             if (k + 1 < n && cb1 != cb) {
                 load_x(cb1);
                 pin_x();
@@ -706,7 +762,7 @@ void k_gemv_wave(const WaveGroup g, const void* __restrict__ x, const WaveShape 
             uint32_t pr2 = pr1 + 1, cb2 = cb1;
             if (pr2 == pairs) pr2 = 0, ++cb2;
             load_unit(a, (k + 2) & 31u, min(cb2, sh.nb - 1), k + 2 < n);
-            if (k + 1 < n) process(b, k + 1, cb1, pr1);
+            if (k + 1 < n) process(b, cb1, pr1);
             cb = cb2, pr = pr2;
             if (k + 2 < n && cb2 != cb1) {
                 load_x(cb2);
@@ -753,20 +809,22 @@ __global__ __launch_bounds__(kDecodeWaves * 64, 4) void k_decode_wave(Desc d, ui
         o_start = d.offsets[b0 + lane];
         o_end = d.offsets[b0 + lane + 1];
     }
-    auto weights = [&](uint32_t c) { return min(1024u, d.cols - c * 1024); };
+    auto size_of = [&](uint32_t c) { return block_size(P, min(1024u, d.cols - c * 1024)); };
     auto load = [&](uint32_t k, uint32_t c, bool live) {
-        const WaveStage s = wave_load<P>(d.data, __builtin_amdgcn_readlane(o_start, k & 63u),
-                                         __builtin_amdgcn_readlane(o_end, k & 63u), weights(c), live, lane);
+        const uint32_t start = __builtin_amdgcn_readlane(o_start, k & 63u);
+        const WaveStage s = wave_load<P>(d.data, start, (int32_t)(__builtin_amdgcn_readlane(o_end, k & 63u) - start),
+                                         size_of(c), live, lane);
         __builtin_amdgcn_sched_barrier(0);
         return s;
     };
     auto finish = [&](const WaveStage& s, uint32_t k, uint32_t row, uint32_t c) {
         uint32_t hi[1][4], lo[1][4], wp[8];
-        const uint32_t w = weights(c);
+        const BlockSize z = size_of(c);
+        const uint32_t w = z.n;
         const WaveStage st[1] = {s};
         const uint32_t start[1] = {(uint32_t)__builtin_amdgcn_readlane(o_start, k)};
-        const uint32_t end[1] = {(uint32_t)__builtin_amdgcn_readlane(o_end, k)};
-        wave_decode<P, 1>(tab, ex, st, d.data, d.table, start, end, w, lane, hi, lo);
+        const int32_t len[1] = {(int32_t)(__builtin_amdgcn_readlane(o_end, k) - start[0])};
+        wave_decode<P, 1>(tab, ex, st, d.data, d.table, start, len, z, lane, hi, lo);
         wave_pairs(hi[0], lo[0], wp);
         uint16_t* dst = out + (uint64_t)row * d.cols + c * 1024 + 16 * lane;
         if (wide && 16 * lane + 16 <= w) {
