@@ -17,12 +17,14 @@
 //                     sums, radix_kernel_gpu.py:639-668) and the decode
 //                     (each block's bits stored instead of the products)
 //   k_gemv_gulp       the same for gulp (2, 2, 4, 8) streams
-//                     (radix_kernel_gpu.py:292-392); M = 8 in quad units; a
-//                     decode mode
+//                     (radix_kernel_gpu.py:292-392): M = 8, in quad units,
+//                     and at M <= 4 rows too long for the wave kernel's sums
+//                     and the matrix policy's quad units; a decode mode
 //   k_gemv_wave, k_decode_wave (wave_kernels.h)
-//                     the GEMV and the decode of 1024-weight blocks the
-//                     sip and gulp kernels do not take: ragged columns, the
-//                     balanced profile, fp32 activations
+//                     the GEMV of gulp at M <= 4, and the GEMV and the
+//                     decode of 1024-weight blocks the sip and gulp kernels
+//                     do not take: ragged columns, the balanced profile,
+//                     fp32 activations
 //   k_gemv_narrow     a raw row-major bf16 weight against M <= 8 rows
 //                     (radix_ops.gemv_narrow, radix_ops.py:177-249)
 //
@@ -2324,6 +2326,21 @@ int wave_takes(const dmx_radix_tensor* t) {
     return fast_policy() && t->block_size == 1024 && fast_directory(t) ? wave_profile(t->n_widths, t->widths) : -1;
 }
 
+// Whether the wave kernel goes before the sip or gulp kernel for this tensor:
+// gulp at up to 4 rows, unless the matrix policy puts 3 and 4 in quad units.
+// Its byte decode takes fewer instructions than k_gemv_gulp's, which is bound
+// by issue there. Measured, graphs over rotated copies, k_gemv_gulp -> wave
+// (us): the 32B-class MLP at M = 1 131.2 -> 114.6; the Linears of a
+// 4096-wide layer (12288 inner) at M = 1, 2, 4 79.9 -> 73.3, 86.2 -> 75.3,
+// 101.4 -> 86.3, at M = 8 (quad units) 105.2 -> 110.5; 1024 x 4096 at M = 1
+// 7.9 -> 6.6. sip stays: M = 1 61.0 -> 61.5 on that layer and 5.3 -> 6.0 at
+// 1024 x 4096, M = 4 74.7 -> 76.5, M = 8 90.1 -> 97.8. Rows whose sums do
+// not fit the wave kernel's LDS (over 2048 / M column blocks) run the gulp
+// kernel, in column phases.
+bool wave_first(const dmx_radix_tensor* t, uint32_t m) {
+    return is_gulp(t) && m <= 4 && !(matrix_policy() && m >= 3) && wave_takes(t) >= 0;
+}
+
 // One launch of the wave kernel over n tensors of profile p and equal cols
 // (already checked; kWaveRaw: t->data is the raw weight). Returns 2, having
 // launched nothing, when two rows' sums per column block do not fit the LDS.
@@ -2382,6 +2399,12 @@ int check_gemv_args(const void* x, int x_dtype, uint32_t m, const void* bias, in
 
 int gemv_one(const dmx_radix_tensor* t, const Desc& d, const void* x, int x_dtype, uint32_t m, const void* bias,
              int bias_dtype, void* out, int out_dtype, hipStream_t s, char* err, size_t errn) {
+    const int p = wave_takes(t);
+    const bool first = wave_first(t, m);
+    if (first) {
+        const int rc = launch_wave(p, &t, 1, x, x_dtype, m, &bias, bias_dtype, &out, out_dtype, s, err, errn);
+        if (rc != 2) return rc;
+    }
     if (sip_eligible(t, x, x_dtype, m)) {
         const int rc = launch_sip(&t, 1, x, m, &bias, bias_dtype, &out, out_dtype, s, err, errn);
         if (rc != 2) return rc;
@@ -2390,8 +2413,7 @@ int gemv_one(const dmx_radix_tensor* t, const Desc& d, const void* x, int x_dtyp
         const int rc = launch_gulp(&t, 1, x, m, &bias, bias_dtype, &out, out_dtype, s, err, errn);
         if (rc != 2) return rc;
     }
-    const int p = wave_takes(t);
-    if (p >= 0) {
+    if (p >= 0 && !first) {
         const int rc = launch_wave(p, &t, 1, x, x_dtype, m, &bias, bias_dtype, &out, out_dtype, s, err, errn);
         if (rc != 2) return rc;
     }
@@ -2531,31 +2553,31 @@ extern "C" int dmx_radix_gemv_group(const dmx_radix_tensor* const* tensors, uint
     if (!tensors || !out || n == 0) return fail(err, errn, "empty tensor group");
     Desc d[kGroupMax];
     bool all_sip = n <= (uint32_t)kGroupMax, all_gulp = all_sip;
-    int wave = all_sip ? wave_takes(tensors[0]) : -1;  // the profile they share, none taken by the sip or gulp kernel
+    // the profile they share, each of them the wave kernel's: first, or none taken by the sip or gulp kernel
+    int wave = all_sip ? wave_takes(tensors[0]) : -1;
     for (uint32_t i = 0; i < n; ++i) {
         Desc di;
         if (check_tensor(tensors[i], di, err, errn)) return 1;
         if (tensors[i]->cols != tensors[0]->cols) return fail(err, errn, "a tensor group must share cols (one activation)");
         if (check_gemv_args(x, x_dtype, m, bias ? bias[i] : nullptr, bias_dtype, out[i], out_dtype, err, errn))
             return 1;
-        all_sip = all_sip && sip_eligible(tensors[i], x, x_dtype, m);
-        all_gulp = all_gulp && gulp_eligible(tensors[i], x, x_dtype, m);
-        if (sip_eligible(tensors[i], x, x_dtype, m) || gulp_eligible(tensors[i], x, x_dtype, m) ||
-            wave_takes(tensors[i]) != wave)
-            wave = -1;
+        const bool sip = sip_eligible(tensors[i], x, x_dtype, m), gulp = gulp_eligible(tensors[i], x, x_dtype, m);
+        all_sip = all_sip && sip;
+        all_gulp = all_gulp && gulp;
+        if (wave_takes(tensors[i]) != wave || ((sip || gulp) && !wave_first(tensors[i], m))) wave = -1;
         if (i < (uint32_t)kGroupMax) d[i] = di;
     }
     hipStream_t s = static_cast<hipStream_t>(stream);
+    if (wave >= 0) {
+        const int rc = launch_wave(wave, tensors, n, x, x_dtype, m, bias, bias_dtype, out, out_dtype, s, err, errn);
+        if (rc != 2) return rc;
+    }
     if (all_sip) {
         const int rc = launch_sip(tensors, n, x, m, bias, bias_dtype, out, out_dtype, s, err, errn);
         if (rc != 2) return rc;
     }
     if (all_gulp) {
         const int rc = launch_gulp(tensors, n, x, m, bias, bias_dtype, out, out_dtype, s, err, errn);
-        if (rc != 2) return rc;
-    }
-    if (wave >= 0) {
-        const int rc = launch_wave(wave, tensors, n, x, x_dtype, m, bias, bias_dtype, out, out_dtype, s, err, errn);
         if (rc != 2) return rc;
     }
     for (uint32_t i = 0; i < n; ++i) {
@@ -2693,13 +2715,18 @@ extern "C" int dmx_radix_gemv_twin(const uint16_t* w, uint32_t rows, uint32_t co
     const bool fast = fast_policy() && m >= 1 && m <= 8 && x_dtype == DMX_BF16 &&
                       block_size == 1024 && cols % 1024 == 0 && (reinterpret_cast<uintptr_t>(x) & 15u) == 0 &&
                       (reinterpret_cast<uintptr_t>(w) & 15u) == 0;
+    t.data = reinterpret_cast<const uint32_t*>(w);
+    const dmx_radix_tensor* tp = &t;
+    const bool first = wave_first(&t, m);
+    if (first) {
+        const int rc = launch_wave(kWaveRaw, &tp, 1, x, x_dtype, m, &bias, bias_dtype, &out, out_dtype, s, err, errn);
+        if (rc != 2) return rc;
+    }
     if (fast && (is_sip(&t) || is_gulp(&t))) {
         const int rc = launch_raw(w, rows, cols, is_gulp(&t), x, m, bias, bias_dtype, out, out_dtype, s, err, errn);
         if (rc != 2) return rc;
     }
-    if (wave_takes(&t) >= 0) {
-        t.data = reinterpret_cast<const uint32_t*>(w);
-        const dmx_radix_tensor* tp = &t;
+    if (wave_takes(&t) >= 0 && !first) {
         const int rc = launch_wave(kWaveRaw, &tp, 1, x, x_dtype, m, &bias, bias_dtype, &out, out_dtype, s, err, errn);
         if (rc != 2) return rc;
     }

@@ -1,8 +1,8 @@
 // The wave kernels: decode + GEMV (k_gemv_wave) and decode alone
 // (k_decode_wave) for 1024-weight blocks of the three profiles, any column
-// count, any activation type. They serve what the sip and gulp kernels do
-// not take: columns that are not whole blocks, the balanced profile, and
-// fp32 activations. Included by kernels.hip, inside its namespace.
+// count, any activation type. They serve gulp at M <= 4 and what the sip and
+// gulp kernels do not take: columns that are not whole blocks, the balanced
+// profile, and fp32 activations. Included by kernels.hip, inside its namespace.
 //
 // Work split. A workgroup of W waves owns T rows (T even) of one tensor. A
 // unit is one column block of two neighbouring rows; the units, column by
@@ -697,9 +697,15 @@ void k_gemv_wave(const WaveGroup g, const void* __restrict__ x, const WaveShape 
                 const uint32_t c0 = cb * 1024 + 16 * lane, n = sh.cols > c0 ? min(16u, sh.cols - c0) : 0u;
                 const uint16_t* w = reinterpret_cast<const uint16_t*>(data) +
                                     (uint64_t)(r0 + min(2 * pr + j, nrows - 1)) * sh.cols + c0;
+                if (cb * 1024 + 1024 <= sh.cols && (reinterpret_cast<uintptr_t>(data) & 15u) == 0 && sh.cols % 8 == 0) {
+                    const u32x4 q0 = reinterpret_cast<const u32x4*>(w)[0], q1 = reinterpret_cast<const u32x4*>(w)[1];
 #pragma unroll
-                for (uint32_t i = 0; i < 8; ++i)
-                    wp[i] = (2 * i < n ? (uint32_t)w[2 * i] : 0u) | (2 * i + 1 < n ? (uint32_t)w[2 * i + 1] << 16 : 0u);
+                    for (uint32_t i = 0; i < 8; ++i) wp[i] = i < 4 ? q0[i & 3] : q1[i & 3];
+                } else {
+#pragma unroll
+                    for (uint32_t i = 0; i < 8; ++i)
+                        wp[i] = (2 * i < n ? (uint32_t)w[2 * i] : 0u) | (2 * i + 1 < n ? (uint32_t)w[2 * i + 1] << 16 : 0u);
+                }
             }
             if constexpr (XT == kWaveX32) {
                 float w[16];

@@ -107,3 +107,33 @@ def test_a_non_finite_weight_past_the_row_end_is_not_multiplied(cuda):
         for xx in (x, x.to(torch.bfloat16)):
             y = radix_ops.gemv_rows(rt, xx, None, torch.float32).cpu().numpy()[0]
             assert np.all(np.isinf(y[:6])) and np.all(np.isfinite(y[6:])), profile
+
+
+@pytest.mark.parametrize("M,blocks", [(1, 2047), (1, 2049), (3, 512), (4, 513), (2, 4), (4, 1)])
+def test_gulp_rows_at_the_edge_of_the_wave_kernels_sums(cuda, M, blocks):
+    """Whole-block gulp at up to four rows runs the wave kernel while two
+    rows' sums fit it (2048 / M column blocks, M rounded up to a power of
+    two), the gulp kernel beyond; three rows of weights, the second of the
+    last unit missing. The twin follows bit for bit, from a 16-byte-aligned
+    weight and from one that is not."""
+    import torch
+
+    from drinkme_amd import radix_ops, swap
+
+    R, C = 3, 1024 * blocks
+    rng = np.random.default_rng(blocks + M)
+    bits = escape_heavy_bits(rng, (R, C), 0.05)
+    rt = swap.to_device_radix(pack_to_dict(O.pack(bits, "gulp", allow_raw=False), "gulp"), cuda)
+    xb = O.f32_to_bf16_bits(rng.standard_normal((M, C)).astype(np.float32))
+    x = bf16_tensor(xb, cuda)
+    print(f"case wave gulp edge M={M} blocks={blocks}", flush=True)
+    y = radix_ops.gemv_rows(rt, x, None, torch.float32)
+    ref, bound = O.gemv_f64(bits, O.bf16_bits_to_f32(xb))
+    assert np.all(np.abs(y.cpu().numpy().astype(np.float64) - ref) <= bound)
+    if blocks <= 512:  # (past that, the gulp kernel and its twin: test_gpu_twin)
+        buf = torch.empty(R * C + 2, dtype=torch.bfloat16, device=cuda)
+        for start in (0, 2):
+            w = buf[start:start + R * C].view(R, C)
+            w.copy_(bf16_tensor(bits, cuda))
+            twin = dict(swap.to_device_twin(w, widths=rt["widths"], device=cuda), weight=w)
+            assert torch.equal(radix_ops.gemv_rows(twin, x, None, torch.float32), y), start
