@@ -8,9 +8,11 @@ here, at first use, with the path it looked for.
 from __future__ import annotations
 
 import ctypes as ct
+import importlib.machinery
+import importlib.util
 import os
 
-from .build import LIB
+from .build import CALLS, LIB
 
 DMX_BF16 = 0
 DMX_F32 = 1
@@ -96,6 +98,26 @@ def lib():
             raise ImportError(f"{LIB}: ABI version {L.dmx_abi_version()}, expected 1")
         _lib = L
     return _lib
+
+
+_calls = None
+
+
+def calls():
+    """The loaded extension of the launchers' per-call path
+    (csrc/torch_calls.cpp; raises when it is not built)."""
+    global _calls
+    if _calls is None:
+        import torch  # noqa: F401  (the extension links torch's libraries, which this loads)
+
+        lib()
+        if not os.path.exists(CALLS):
+            raise ImportError(f"dmx_calls.so is not built ({CALLS}); run `python -m drinkme_amd.build`")
+        loader = importlib.machinery.ExtensionFileLoader("dmx_calls", CALLS)
+        module = importlib.util.module_from_spec(importlib.util.spec_from_loader("dmx_calls", loader))
+        loader.exec_module(module)
+        _calls = module
+    return _calls
 
 
 def error_buffer():

@@ -8,7 +8,9 @@ with hipcc for gfx950 only, and all linked into one shared library that
 ctypes loads (drinkme_amd/_native.py). Packed-fp32 instructions are
 disabled for the device code (-packed-fp32-ops): hipcc otherwise forms
 v_pk_*_f32 from scalar float code. The host-only command line tool
-lib/dmx_pack (csrc/dmx_pack.cpp) is linked from the same host sources.
+lib/dmx_pack (csrc/dmx_pack.cpp) is linked from the same host sources. The
+launchers' per-call path over torch tensors (csrc/torch_calls.cpp) is a
+CPython extension beside the library, lib/dmx_calls.so, linked to it.
 """
 
 from __future__ import annotations
@@ -17,6 +19,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
@@ -25,6 +28,7 @@ OBJ = os.path.join(HERE, "_build")
 LIBDIR = os.path.join(HERE, "lib")
 LIB = os.path.join(LIBDIR, "libdmx_radix.so")
 CLI = os.path.join(LIBDIR, "dmx_pack")
+CALLS = os.path.join(LIBDIR, "dmx_calls.so")
 INCLUDE = os.path.join(ROOT, "include")
 ARCH = "gfx950"
 
@@ -69,6 +73,17 @@ def build(verbose: bool = False) -> str:
     os.replace(tmp, LIB)
     _run(["g++", "-pthread", *objs, "-o", CLI + ".tmp"], verbose)
     os.replace(CLI + ".tmp", CLI)
+    import torch
+
+    home = os.path.dirname(torch.__file__)
+    dirs = [os.path.join(home, "include"), os.path.join(home, "include", "torch", "csrc", "api", "include"),
+            sysconfig.get_paths()["include"]]
+    _run([*host, "-O2", *(f for d in dirs for f in ("-isystem", d)),
+          f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-shared",
+          os.path.join(CSRC, "torch_calls.cpp"), "-L" + LIBDIR, "-l:" + os.path.basename(LIB),
+          "-L" + os.path.join(home, "lib"), "-ltorch_python", "-ltorch_cpu", "-lc10", "-Wl,-rpath,$ORIGIN",
+          "-o", CALLS + ".tmp"], verbose)
+    os.replace(CALLS + ".tmp", CALLS)
     return LIB
 
 

@@ -443,6 +443,10 @@ class NarrowLinear(torch.nn.Linear):
         return mod
 
     def forward(self, x):
+        if x.is_cuda and x.numel() <= radix_ops.MC_MAX * self.in_features:
+            y = radix_ops.narrow_rows(self.weight, x, self.bias)
+            if y is not None:
+                return y
         rows = x.reshape(-1, self.in_features)
         if x.device.type != "cuda" or rows.shape[0] > radix_ops.MC_MAX:
             return torch.nn.functional.linear(x, self.weight, self.bias)
