@@ -127,14 +127,16 @@ class HostCodec:
     Ops: PLAN fills the tables and the directory and returns the payload's
     word count; ENCODE fills the payload; DECODE writes rows
     [first, first + count) starting at the output pointer it is given;
-    CHECK_PALETTE refuses repeated, out-of-range or padding-dirty tables."""
+    CHECK_PALETTE refuses repeated, out-of-range or padding-dirty tables;
+    COMPARE decodes rows [first, first + count) and returns 1 where they
+    equal those at the pointer it is given, else 0."""
 
     rows: int
     cols: int
     widths: tuple
     _w: np.ndarray = field(init=False, repr=False)
 
-    PLAN, ENCODE, DECODE, CHECK_PALETTE = 0, 1, 2, 3
+    PLAN, ENCODE, DECODE, CHECK_PALETTE, COMPARE = 0, 1, 2, 3, 4
 
     def __post_init__(self):
         self.rows, self.cols = int(self.rows), int(self.cols)
@@ -170,7 +172,7 @@ class HostCodec:
         offsets = np.zeros(self.directory_len, dtype=np.uint32)
         data = np.zeros(self.op(self.PLAN, bits, tables, offsets), dtype=np.uint32)
         self.op(self.ENCODE, bits, tables, offsets, data)
-        if not np.array_equal(self.expand(tables, offsets, data), bits):
+        if not self.op(self.COMPARE, bits, tables, offsets, data, 0, self.rows):
             raise ValueError("native radix: CPU round trip differs from the source bits")
         return tables, offsets, data
 

@@ -85,7 +85,9 @@ uint64_t dmx_radix_pad_words(uint32_t block_size, const uint32_t* widths, uint32
  * the same signature and meaning: op 0 plan (palette tables + directory,
  * *result = payload words), 1 encode, 2 decode rows [first, first + nrows)
  * into the pointer given (row `first` at its start), 3 validate the
- * palette tables. 1024-weight blocks; palettes per region of rg rows x cg
+ * palette tables; and one op more, 4: compare rows [first, first + nrows)
+ * with those at the pointer given, *result = 1 where equal, else 0 (the
+ * encoder's round-trip check, without the decoded copy). 1024-weight blocks; palettes per region of rg rows x cg
  * blocks. Runs on host threads (dmx_set_host_threads). */
 int dmx_radix_native(uint32_t op, void* source_or_output, uint64_t rows, uint64_t cols, uint64_t rg,
                      uint64_t cg, uint32_t mant, uint32_t exponent, const uint32_t* widths, uint32_t count,
