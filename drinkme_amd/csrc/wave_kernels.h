@@ -24,12 +24,14 @@
 // for 284, sip 3584 x 9472 14.3 for 149; gulp fp32 M = 2 q/k/v of 10240 x
 // 5120 23.8 for 326; balanced q/k/v of 6144 x 4096 12.8 for 145.
 //
-// The decode works on bytes. A table entry holds four exponent bytes and a
-// v_perm selector over (four consecutive bytes of the next tier's
-// exponents, the entry's own four): byte k is k where weight k resolved in
-// this tier, 4 + its rank among the group's escapes where it did not. One
-// v_perm so completes a group, and bit 2 of a selector byte is the escape
-// flag, which a masked popcount counts.
+// The decode works on bytes. A table entry holds the exponent bytes of the
+// weights that resolved in this tier and a v_perm selector over (four
+// consecutive bytes of the next tier's exponents, the entry's own four): byte
+// k is 4 + the weight's rank among the group's e escapes, or e + its rank
+// among the others (whose exponents lie at those bytes of the entry). One
+// v_perm so completes a group, and with the own bytes placed so the bits set
+// in the selector are 4 + e for every pattern: one popcount, unmasked, counts
+// the escapes, and its 4 a group goes into the windows' immediate offsets.
 //   tier 0   lane l owns weights 16l .. 16l + 15, four table lookups;
 //   tier 1   (balanced, gulp) lane l resolves the block's tier-0 escapes
 //            8l .. 8l + 7 from the tail words, which a wave keeps in LDS,
@@ -85,6 +87,9 @@ struct WaveTables {
 // each with one word more; the tier-1 exponent bytes (512 and a window's
 // overhang) and the tier-2 ones (128 and the overhang).
 constexpr uint32_t kExTerm = 0, kExTail = 66, kExT1 = 132, kExT2 = kExT1 + 130;
+// (in front of the exchanges, in uint2: a window's address before its offset
+// is up to 12 bytes short of it)
+constexpr uint32_t kExHead = 2;
 constexpr uint32_t wave_exchange(int P) {
     return P == kWaveSip ? kExTail : P == kWaveBalanced ? kExT2 : P == kWaveGulp ? kExT2 + 34 : 0u;
 }
@@ -96,47 +101,52 @@ __device__ __forceinline__ uint32_t rotate_bytes(uint32_t v) {
     return ((v >> 1) & 0x7F7F7F7Fu) | ((v << 7) & 0x80808080u);
 }
 
-// Two words of LDS from byte address `at` on, `at` rounded down to a word,
-// and the four bytes from `at` in them. (One unaligned ds_read_b32 instead
+// Two words of LDS from byte address `at` + `past` (a multiple of 4) on, `at`
+// rounded down to a word, and the four bytes from `at` in them. (One unaligned ds_read_b32 instead
 // stalls the LDS for about 60 cycles a wave: the 9472 x 3584 gate/up launch
 // took 45.6 us with it, 28.8 us without.)
 typedef const __attribute__((address_space(3))) uint32_t* lds_words;
 __device__ __forceinline__ uint32_t lds_address(const void* p) { return (uint32_t)(uintptr_t)(lds_ptr)p; }
-__device__ __forceinline__ uint2 lds_window(uint32_t at) {
+__device__ __forceinline__ uint2 lds_window(uint32_t at, uint32_t past = 0) {
     const lds_words p = (lds_words)(uintptr_t)(at & ~3u);
-    return make_uint2(p[0], p[1]);
+    return make_uint2(p[past / 4], p[past / 4 + 1]);
 }
 __device__ __forceinline__ uint32_t window_bytes(uint2 w, uint32_t at) { return __builtin_amdgcn_alignbyte(w.y, w.x, at); }
 
-// Entry of four codes c[k] < 2^w, exponents from the run `pal` of the padded
-// tables (the escape code reads its zero pad byte).
+// Entry of N codes c[k] < 2^w (two: the selector's upper bytes are 0),
+// exponents from the run `pal` of the padded tables.
 template <uint32_t w, uint32_t N>
 __device__ __forceinline__ uint2 wave_entry(uint32_t i, const uint32_t (&pal)[4]) {
-    uint32_t e = 0, sel = 0x03020100u, r = 4;
+    uint32_t e = 0, sel = 0, r = 4, own = 0;
+#pragma unroll
+    for (uint32_t k = 0; k < N; ++k) own += ((i >> (w * k)) & ((1u << w) - 1u)) == (1u << w) - 1u;
 #pragma unroll
     for (uint32_t k = 0; k < N; ++k) {
         const uint32_t c = (i >> (w * k)) & ((1u << w) - 1u);
         uint32_t b = __builtin_amdgcn_perm(pal[1], pal[0], c & 7u);
         if (w == 4) b = c & 8u ? __builtin_amdgcn_perm(pal[3], pal[2], c & 7u) : b;
-        e |= (b & 0xFFu) << (8 * k);  // (rotated bytes, as pal's are)
-        if (c == (1u << w) - 1u) sel ^= (k ^ r++) << (8 * k);
+        const bool esc = c == (1u << w) - 1u;
+        e |= esc ? 0u : (b & 0xFFu) << (8 * own);  // (rotated bytes, as pal's are)
+        sel |= (esc ? r : own) << (8 * k);
+        r += esc;
+        own += !esc;
     }
     return make_uint2(e, sel);
 }
 
 // The 4096 entries of four 3-bit codes (palette words p0, p1): entries 8h ..
-// 8h + 7 share the upper three codes, and only c0 = 7 (an escape) moves
-// their ranks.
+// 8h + 7 share the upper three codes, so but for c0 = 7 (an escape) their
+// selector and the byte, `at`, of c0's exponent.
 __device__ __forceinline__ void wave_table3(uint2* tab, uint32_t p0, uint32_t p1, uint32_t threads) {
     const uint32_t pal[4] = {p0, p1, 0, 0};
     for (uint32_t h = threadIdx.x; h < 512; h += threads) {
         const uint2 e = wave_entry<3, 4>(8 * h, pal), esc = wave_entry<3, 4>(8 * h + 7, pal);
-        const uint32_t up = e.x & 0xFFFFFF00u;
+        const uint32_t at = 8 * (e.y & 3u), up = e.x & ~(0xFFu << at);
 #pragma unroll
         for (uint32_t c = 0; c < 8; c += 2) {
             const uint32_t two = c < 4 ? p0 >> (8 * c) : p1 >> (8 * (c - 4));
-            const uint2 odd = c == 6 ? esc : make_uint2(up | ((two >> 8) & 0xFFu), e.y);
-            *reinterpret_cast<uint4*>(tab + 8 * h + c) = make_uint4(up | (two & 0xFFu), e.y, odd.x, odd.y);
+            const uint2 odd = c == 6 ? esc : make_uint2(up | ((two >> 8) & 0xFFu) << at, e.y);
+            *reinterpret_cast<uint4*>(tab + 8 * h + c) = make_uint4(up | (two & 0xFFu) << at, e.y, odd.x, odd.y);
         }
     }
 }
@@ -252,10 +262,8 @@ __device__ __forceinline__ uint32_t keep_bits(uint32_t codes, int32_t bits, int3
     return __builtin_amdgcn_ubfe(codes, 0, (uint32_t)min(max(bits, 0), most));
 }
 
-// Escapes of an entry, added to n.
-__device__ __forceinline__ uint32_t add_escapes(uint2 e, uint32_t n) {
-    return (uint32_t)__builtin_popcount(e.y & 0x04040404u) + n;
-}
+// Escapes of an entry of four codes, and 4 (of two codes, and 1), added to n.
+__device__ __forceinline__ uint32_t add_escapes(uint2 e, uint32_t n) { return (uint32_t)__builtin_popcount(e.y) + n; }
 
 // Completes an entry from the next tier's four exponent bytes.
 __device__ __forceinline__ uint32_t complete(uint2 e, uint32_t next) { return __builtin_amdgcn_perm(next, e.x, e.y); }
@@ -277,7 +285,7 @@ __device__ __forceinline__ void wave_decode(const uint2* tab, uint32_t* ex, cons
     constexpr uint32_t stride = wave_exchange(P);
     const uint32_t ex_at = lds_address(ex);
     uint2 e[R][4];
-    uint32_t c[R][4];  // escapes of groups 0 .. g
+    uint32_t c[R][4];  // escapes of groups 0 .. g, less 4 (3 - g)
     int32_t tail[R], bad = 0;  // (bad: negative once a limit is passed; every quantity is far below 2^31)
     uint32_t T[R][2];
 #pragma unroll
@@ -330,7 +338,7 @@ __device__ __forceinline__ void wave_decode(const uint2* tab, uint32_t* ex, cons
     uint32_t cnt[R];
 #pragma unroll
     for (int j = 0; j < R; ++j) {
-        c[j][0] = add_escapes(e[j][0], 0);
+        c[j][0] = add_escapes(e[j][0], ~15u);
 #pragma unroll
         for (int g = 1; g < 4; ++g) c[j][g] = add_escapes(e[j][g], c[j][g - 1]);
         cnt[j] = c[j][3];
@@ -343,7 +351,7 @@ __device__ __forceinline__ void wave_decode(const uint2* tab, uint32_t* ex, cons
     } else {
         // lane l: the block's tier-1 codes 8l .. 8l + 7
         constexpr uint32_t w = wave_width(P, 1);
-        uint32_t w1[R], g0[R], q1[R], n2[R];
+        uint32_t w1[R], g0[R], q1[R], n2[R];  // (g0: escapes of the first group, less 4)
         uint2 a[R][2];
         uint2 win[R][2];
         // the two groups' windows in the exponent bytes at byte `at` of the
@@ -352,7 +360,7 @@ __device__ __forceinline__ void wave_decode(const uint2* tab, uint32_t* ex, cons
         auto windows = [&](int j, uint32_t at) {
             p1[j] = q1[j] + at;
             win[j][0] = lds_window(p1[j]);
-            win[j][1] = lds_window(p1[j] + g0[j]);
+            win[j][1] = lds_window(p1[j] + g0[j], 4);
         };
         auto finish = [&]() {
             __builtin_amdgcn_sched_barrier(0);
@@ -381,7 +389,7 @@ __device__ __forceinline__ void wave_decode(const uint2* tab, uint32_t* ex, cons
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int j = 0; j < R; ++j) {
-            g0[j] = add_escapes(a[j][0], 0);
+            g0[j] = add_escapes(a[j][0], ~7u);
             cnt[j] = add_escapes(a[j][1], g0[j]);
         }
         scan(cnt, q1, n2);
@@ -405,7 +413,7 @@ __device__ __forceinline__ void wave_decode(const uint2* tab, uint32_t* ex, cons
             }
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int j = 0; j < R; ++j) cnt[j] = add_escapes(b[j], 0);
+            for (int j = 0; j < R; ++j) cnt[j] = add_escapes(b[j], ~0u);
             if (__builtin_amdgcn_ballot_w64((cnt[0] | cnt[R - 1]) != 0) != 0) {
                 uint32_t q2[R], n3[R];
                 scan(cnt, q2, n3);
@@ -435,7 +443,7 @@ __device__ __forceinline__ void wave_decode(const uint2* tab, uint32_t* ex, cons
         q[j] += ex_at + 4 * (j * stride + below);
         win[j][0] = lds_window(q[j]);
 #pragma unroll
-        for (int g = 1; g < 4; ++g) win[j][g] = lds_window(c[j][g - 1] += q[j]);
+        for (int g = 1; g < 4; ++g) win[j][g] = lds_window(c[j][g - 1] += q[j], 16 - 4 * g);
     }
     __builtin_amdgcn_sched_barrier(0);
     uint32_t E[R][4];
@@ -565,7 +573,9 @@ constexpr uint32_t wave_occ(int P, int M, int XT) {
 }
 constexpr uint32_t kDecodeWaves = 8;
 // static LDS of the wave kernel
-constexpr size_t wave_lds(int P, uint32_t W) { return 8 * ((size_t)W * wave_exchange(P) + WaveTables::entries(P)); }
+constexpr size_t wave_lds(int P, uint32_t W) {
+    return 8 * (kExHead + (size_t)W * wave_exchange(P) + WaveTables::entries(P));
+}
 static_assert(wave_exchange(kWaveSip) % 2 == 0 && wave_exchange(kWaveBalanced) % 2 == 0 && wave_exchange(kWaveGulp) % 2 == 0,
               "the exchanges are whole uint2");
 
@@ -574,8 +584,8 @@ __global__ __launch_bounds__(wave_waves(P, M, XT) * 64, wave_occ(P, M, XT))
 void k_gemv_wave(const WaveGroup g, const void* __restrict__ x, const WaveShape sh) {
     constexpr uint32_t W = wave_waves(P, M, XT);
     constexpr int XR = XT == kWaveX32 ? 16 : 8;  // activation registers per row
-    __shared__ __align__(16) uint2 lds[W * wave_exchange(P) + WaveTables::entries(P)];
-    uint2* tab = lds + W * wave_exchange(P);
+    __shared__ __align__(16) uint2 lds[kExHead + W * wave_exchange(P) + WaveTables::entries(P)];
+    uint2* tab = lds + kExHead + W * wave_exchange(P);
     extern __shared__ __align__(16) uint8_t lds_dyn[];
     float* red = reinterpret_cast<float*>(lds_dyn);
 
@@ -594,7 +604,7 @@ void k_gemv_wave(const WaveGroup g, const void* __restrict__ x, const WaveShape 
     const uint32_t pairs = (nrows + 1) / 2, units = pairs * sh.nb;
     const uint32_t u0 = units * wv / W, u1 = units * (wv + 1) / W;
     const uint32_t first = r0 * sh.nb;  // the tile's first block
-    uint32_t* ex0 = reinterpret_cast<uint32_t*>(lds) + wv * 2 * wave_exchange(P);
+    uint32_t* ex0 = reinterpret_cast<uint32_t*>(lds + kExHead) + wv * 2 * wave_exchange(P);
 
     uint32_t xr[M][XR];
     // (through one buffer resource, a row's start the scalar offset: 128-bit
@@ -805,11 +815,11 @@ template <int P>
 __global__ __launch_bounds__(kDecodeWaves * 64, 4) void k_decode_wave(Desc d, uint16_t* __restrict__ out, uint32_t run,
                                                                      uint32_t wide) {
     constexpr uint32_t W = kDecodeWaves;
-    __shared__ __align__(16) uint2 lds[W * wave_exchange(P) / 2 + WaveTables::entries(P)];
-    uint2* tab = lds + W * wave_exchange(P) / 2;
+    __shared__ __align__(16) uint2 lds[kExHead + W * wave_exchange(P) / 2 + WaveTables::entries(P)];
+    uint2* tab = lds + kExHead + W * wave_exchange(P) / 2;
     const uint32_t wv = wave_id(), lane = lane_id(), blocks = d.rows * d.nb;
     const uint32_t b0 = min(blocks, (blockIdx.x * W + wv) * run), n = min(run, blocks - b0);
-    uint32_t* ex = reinterpret_cast<uint32_t*>(lds) + wv * wave_exchange(P);
+    uint32_t* ex = reinterpret_cast<uint32_t*>(lds + kExHead) + wv * wave_exchange(P);
     uint32_t o_start = 0, o_end = 0;
     if (lane < n) {
         o_start = d.offsets[b0 + lane];
