@@ -17,12 +17,15 @@
 //
 // What bounds it: for launches of a few units a wave, the 6 us before and
 // after them (the directory's round trip, the first payload, the tables);
-// for longer ones the payload's stream and the VALU (80 instructions a sip
-// block at M = 1 bf16, 95 to 105 with more tiers, 16 M + 16 more for fp32
+// for longer ones the payload's stream and the VALU (76 instructions a sip
+// block at M = 1 bf16, 88 to 98 with more tiers, 16 M + 16 more for fp32
 // products). Measured, one launch, against k_gemv_generic, which scans over
 // a workgroup with two barriers a tier: sip 2 x 9472 x 3584 (ragged) 21.2 us
 // for 284, sip 3584 x 9472 14.3 for 149; gulp fp32 M = 2 q/k/v of 10240 x
-// 5120 23.8 for 326; balanced q/k/v of 6144 x 4096 12.8 for 145.
+// 5120 23.8 for 326; balanced q/k/v of 6144 x 4096 12.8 for 145. Against
+// k_gemv_gulp: wave_first (kernels.hip). More waves measured slower at M = 1:
+// 10-wave workgroups at five a SIMD 113 -> 139 us on the gulp MLP of 25600 x
+// 5120, 12-wave ones at six (80 registers, spilled) 171.
 //
 // The decode works on bytes. A table entry holds the exponent bytes of the
 // weights that resolved in this tier and a v_perm selector over (four
