@@ -2554,7 +2554,7 @@ extern "C" int dmx_radix_gemv_group(const dmx_radix_tensor* const* tensors, uint
     Desc d[kGroupMax];
     bool all_sip = n <= (uint32_t)kGroupMax, all_gulp = all_sip;
     // the profile they share, each of them the wave kernel's: first, or none taken by the sip or gulp kernel
-    int wave = all_sip ? wave_takes(tensors[0]) : -1;
+    int wave = -1;
     for (uint32_t i = 0; i < n; ++i) {
         Desc di;
         if (check_tensor(tensors[i], di, err, errn)) return 1;
@@ -2564,6 +2564,7 @@ extern "C" int dmx_radix_gemv_group(const dmx_radix_tensor* const* tensors, uint
         const bool sip = sip_eligible(tensors[i], x, x_dtype, m), gulp = gulp_eligible(tensors[i], x, x_dtype, m);
         all_sip = all_sip && sip;
         all_gulp = all_gulp && gulp;
+        if (i == 0 && n <= (uint32_t)kGroupMax) wave = wave_takes(tensors[0]);
         if (wave_takes(tensors[i]) != wave || ((sip || gulp) && !wave_first(tensors[i], m))) wave = -1;
         if (i < (uint32_t)kGroupMax) d[i] = di;
     }

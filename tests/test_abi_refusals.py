@@ -90,6 +90,21 @@ def test_group_refusals():
     assert st != 0 and b"share cols" in err.value
 
 
+@pytest.mark.parametrize("n,null", [(1, 0), (2, 0), (2, 1), (5, 0), (5, 4)])
+def test_a_group_with_a_null_descriptor_is_refused(n, null):
+    from drinkme_amd import _native
+
+    L = _native.lib()
+    err = _native.error_buffer()
+    ts = [_tensor() for _ in range(n)]
+    arr = (ct.POINTER(_native.RadixTensor) * n)(*[ct.pointer(t) for t in ts])
+    arr[null] = ct.POINTER(_native.RadixTensor)()
+    outs = (ct.c_void_p * n)(*[FAKE] * n)
+    st = L.dmx_radix_gemv_group(arr, n, FAKE, _native.DMX_BF16, 1, None, 0, outs, _native.DMX_BF16, None, err,
+                                len(err))
+    assert st != 0 and b"null tensor descriptor" in err.value
+
+
 PROBE_CASES = [
     ("null data", {"data": None}, b"null data or sink"),
     ("null sink", {"sink": None}, b"null data or sink"),
