@@ -89,6 +89,16 @@ __device__ __forceinline__ uint32_t field(const uint32_t* s, uint32_t i, uint32_
 __device__ __forceinline__ uint32_t wave_id() { return __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); }
 __device__ __forceinline__ uint32_t lane_id() { return threadIdx.x & 63u; }
 
+// Between LDS writes of a wave's lanes and reads of them by other lanes, or in
+// another type, and before the words are written again: the compiler moves no
+// memory access over it. It costs no instruction: the hardware completes a
+// wave's LDS operations in order. (wave_barrier alone is no memory operation
+// to the optimiser, and two types are allowed to pass each other.)
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
 // Inclusive prefix sum over the 64 lanes: row_shr 1, 2, 4, 8 inside each
 // 16-lane row, then row_bcast 15 / 31 carry the rows' totals forward.
 __device__ __forceinline__ uint32_t wave_scan_incl(uint32_t v) {
@@ -1680,7 +1690,7 @@ void k_gemv_gulp(const SipGroup g, const uint16_t* __restrict__ x, const SipShap
                 if (tb) eb = ta ? (tw >> 8) & 0xFFu : tw & 0xFFu;
             }
             reinterpret_cast<uint16_t*>(x2)[lane] = (uint16_t)(ea | (eb << 8));
-            __builtin_amdgcn_wave_barrier();
+            wave_lds_sync();
             // each lane's window of 8 exponent bytes from rank q1, placed by the
             // selector of (its tier-1 escapes before the group, the group's m1)
             const uint32_t kq = q1 >> 2;
@@ -1713,7 +1723,7 @@ void k_gemv_gulp(const SipGroup g, const uint16_t* __restrict__ x, const SipShap
             DMX_T2(E3, M == 1 ? sg3 : DMX_SEL(P3, p3))
 #undef DMX_T2
 #undef DMX_SEL
-            __builtin_amdgcn_wave_barrier();
+            wave_lds_sync();
         }
         const uint32_t L0 = s0.lit.x, L1 = s0.lit.y, L2 = s0.lit.z, L3 = s0.lit.w;
         uint32_t wp[8];

@@ -305,6 +305,7 @@ __device__ __forceinline__ void wave_decode(const uint2* tab, uint32_t* ex, cons
             T[j][0] = s[j].t0.x;
         }
     }
+    wave_lds_sync();
     if (z.n < 1024) {
         const int32_t bits = ((int32_t)z.n - 16 * (int32_t)lane) * (int32_t)wave_width(P, 0);
 #pragma unroll
@@ -429,7 +430,7 @@ __device__ __forceinline__ void wave_decode(const uint2* tab, uint32_t* ex, cons
             }
 #pragma unroll
             for (int j = 0; j < R; ++j) reinterpret_cast<uint16_t*>(ex + j * stride + kExT2)[lane] = (uint16_t)b[j].x;
-            __builtin_amdgcn_wave_barrier();
+            wave_lds_sync();
 #pragma unroll
             for (int j = 0; j < R; ++j) windows(j, ex_at + 4 * (j * stride + kExT2));
         }
@@ -437,7 +438,7 @@ __device__ __forceinline__ void wave_decode(const uint2* tab, uint32_t* ex, cons
 #pragma unroll
         for (int j = 0; j < R; ++j)
             *reinterpret_cast<uint2*>(ex + j * stride + kExT1 + 2 * lane) = make_uint2(a[j][0].x, a[j][1].x);
-        __builtin_amdgcn_wave_barrier();
+        wave_lds_sync();
         below = kExT1;
     }
     uint2 win[R][4];
@@ -456,7 +457,7 @@ __device__ __forceinline__ void wave_decode(const uint2* tab, uint32_t* ex, cons
 #pragma unroll
         for (int g = 1; g < 4; ++g) E[j][g] = complete(e[j][g], window_bytes(win[j][g], c[j][g - 1]));
     }
-    __builtin_amdgcn_wave_barrier();
+    wave_lds_sync();
     if (__builtin_expect(bad < 0, 0)) {
 #pragma unroll 1
         for (int j = 0; j < R; ++j) {
