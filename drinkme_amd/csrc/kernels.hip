@@ -2344,7 +2344,10 @@ int wave_takes(const dmx_radix_tensor* t) {
 // 4096-wide layer (12288 inner) at M = 1, 2, 4 79.9 -> 73.3, 86.2 -> 75.3,
 // 101.4 -> 86.3, at M = 8 (quad units) 105.2 -> 110.5; 1024 x 4096 at M = 1
 // 7.9 -> 6.6. sip stays: M = 1 61.0 -> 61.5 on that layer and 5.3 -> 6.0 at
-// 1024 x 4096, M = 4 74.7 -> 76.5, M = 8 90.1 -> 97.8. Rows whose sums do
+// 1024 x 4096, M = 4 74.7 -> 76.5, M = 8 90.1 -> 97.8. Where rows differ in
+// scale, so that blocks leave either kernel's fast path (12288 x 4096, M = 1,
+// rows scaled by a lognormal of sigma 0.3, 0.5, 1.0): 48.9 -> 22.1, 83.0 ->
+// 27.0, 123.3 -> 42.9. Rows whose sums do
 // not fit the wave kernel's LDS (over 2048 / M column blocks) run the gulp
 // kernel, in column phases.
 bool wave_first(const dmx_radix_tensor* t, uint32_t m) {

@@ -46,10 +46,9 @@
 // a level for both rows of a unit (counts of at most 1024, 16 bits each).
 // The two rows' decodes run side by side with no branch between them, so one
 // row's LDS round trips cover the other's (decoded one after the other, the
-// waves waited 44% of their time). A unit with a block outside the limits
-// (more than 512 tier-0 or 128 tier-1 escapes, a tail of more than 64
-// words, streams cut short) takes wave_exact, which reads every field from
-// memory as decode_block does.
+// waves waited 44% of their time). A block outside the limits (more than 512
+// tier-0 or 128 tier-1 escapes, a tail of more than 64 words, streams cut
+// short) takes wave_wide, which reads its streams from memory.
 
 enum WaveProfile { kWaveSip = 0, kWaveBalanced = 1, kWaveGulp = 2, kWaveRaw = 3 };
 
@@ -215,50 +214,6 @@ __device__ __forceinline__ WaveStage wave_load(const uint32_t* data, uint32_t st
     return s;
 }
 
-// The lane's 16 exponent bytes (rotated) with every field read from memory, as
-// decode_block reads them (any escape counts, streams of any length).
-template <int P>
-__device__ void wave_exact(const uint32_t* data, const uint8_t* pal, uint32_t start, uint32_t end, uint32_t n,
-                           uint32_t lane, uint32_t (&E)[4]) {
-    const uint32_t valid = n > 16 * lane ? min(16u, n - 16 * lane) : 0u;
-    uint32_t active = (1u << valid) - 1u;
-    uint64_t elo = 0, ehi = 0;  // exponent byte of weight i: byte i & 7 of (i < 8 ? elo : ehi)
-    auto place = [&](int i, uint32_t e) {
-        const uint64_t v = (uint64_t)e << (8 * (i & 7));
-        if (i < 8)
-            elo |= v;
-        else
-            ehi |= v;
-    };
-    uint32_t pos = start + words_for(n, 8);
-#pragma unroll
-    for (uint32_t j = 0; j < wave_tiers(P); ++j) {
-        const uint32_t w = wave_width(P, j), esc = (1u << w) - 1u;
-        const uint32_t cnt = __builtin_popcount(active), inc = wave_scan_incl(cnt);
-        uint32_t r = inc - cnt;
-#pragma unroll 1
-        for (int i = 0; i < 16; ++i) {
-            if (!((active >> i) & 1u)) continue;
-            const uint32_t code = field(data + pos, r++, w);
-            if (code == esc) continue;
-            place(i, pal[wave_pal_byte(P, j) + code]);
-            active &= ~(1u << i);
-        }
-        pos += words_for(__builtin_amdgcn_readlane(inc, 63), w);
-    }
-    const uint32_t cnt = __builtin_popcount(active), inc = wave_scan_incl(cnt);
-    uint32_t r = inc - cnt;
-    if (end > pos) {  // (the terminal is read only where the directory gives the block words for it)
-#pragma unroll 1
-        for (int i = 0; i < 16; ++i)
-            if ((active >> i) & 1u) place(i, field(data + pos, r++, 8));
-    }
-    E[0] = rotate_bytes((uint32_t)elo);
-    E[1] = rotate_bytes((uint32_t)(elo >> 32));
-    E[2] = rotate_bytes((uint32_t)ehi);
-    E[3] = rotate_bytes((uint32_t)(ehi >> 32));
-}
-
 // The first `bits` (clamped to 0 .. most < 32) bits of codes: those past the
 // stream's end read as 0, which no tier takes for an escape.
 __device__ __forceinline__ uint32_t keep_bits(uint32_t codes, int32_t bits, int32_t most) {
@@ -271,6 +226,131 @@ __device__ __forceinline__ uint32_t add_escapes(uint2 e, uint32_t n) { return (u
 // Completes an entry from the next tier's four exponent bytes.
 __device__ __forceinline__ uint32_t complete(uint2 e, uint32_t next) { return __builtin_amdgcn_perm(next, e.x, e.y); }
 
+// The farthest word past a block's start that any of its streams reaches.
+constexpr uint32_t wave_bound(int P) {
+    uint32_t b = 2 * 256;  // literals, terminal
+    for (uint32_t j = 0; j < wave_tiers(P); ++j) b += 32 * wave_width(P, j);
+    return b;
+}
+
+// The lane's 16 exponent bytes (rotated) of a block outside the limits, with
+// the meaning of decode_block: any escape counts, streams of any length, read
+// from memory. Lane l owns codes 16l .. 16l + 15 of every tier, two words of
+// them at most, so a tier costs one round trip to memory (tier 0 and tier 1
+// together: their places are known), its lookups and one scan; each level's
+// bytes go down through the exchange, whose first 258 words serve the levels
+// in turn, and the terminal's are read in place. Such blocks are ordinary
+// where one palette serves rows of different scale: of 12288 x 4096 N(0, 0.02)
+// gulp weights with rows scaled by a lognormal of sigma 0.3, 0.5, 1.0, M = 1,
+// the launch takes 22, 27, 43 us (unscaled 18); reading one field at a time,
+// both rows of a unit together, took 78, 142, 226. The loads go through a
+// buffer resource that ends one word past the streams' bound, which the pad
+// covers: the bound counts from the block's first word.
+template <int P>
+__device__ __forceinline__ void wave_wide(const uint2* tab, uint32_t* ex, const uint32_t* data, uint32_t start,
+                                          uint32_t end, const BlockSize& z, uint32_t lane, uint32_t (&E)[4]) {
+    const auto r = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint32_t*>(data + start), 0, 4 * (wave_bound(P) + 1),
+                                                     0x00020000);
+    const uint32_t len = end - start;
+    uint32_t pos = z.fixed;
+    asm volatile("" : "+v"(lane));  // (else its multiples are kept in registers over the unit loop)
+    auto words = [&](uint32_t byte) {  // two words of the block, from the byte on (a multiple of 4)
+        return __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(r, byte, 0, 0));
+    };
+    auto load = [&](uint32_t at, uint32_t n, uint32_t w, uint32_t (&t)[2]) {  // 16 w-bit codes of n at word `at`
+        const uint32_t bit = 16 * w * lane;
+        const u32x2 v = words(16 * lane < n ? 4 * (at + (bit >> 5)) : 0x80000000u);
+        const uint64_t all = ((uint64_t)v.y << 32 | v.x) >> (bit & 31u);
+        t[0] = (uint32_t)all;
+        t[1] = (uint32_t)(all >> 32);
+    };
+    auto keep = [&](uint32_t n, uint32_t w, uint32_t (&t)[2]) {
+        const int32_t bits = ((int32_t)n - 16 * (int32_t)lane) * (int32_t)w;
+        t[0] = bits >= 32 ? t[0] : keep_bits(t[0], bits, 31);
+        t[1] = bits >= 64 ? t[1] : keep_bits(t[1], bits - 32, 31);
+    };
+    auto group = [&](const uint2* t, uint32_t w, const uint32_t (&c)[2], int g) {  // four codes' entry
+        const uint64_t v = (uint64_t)c[1] << 32 | c[0];
+        return t[(uint32_t)(v >> (4 * w * g)) & ((1u << (4 * w)) - 1u)];
+    };
+    // the rank of the lane's first escape among a tier's (four groups of codes
+    // c), and how many there are
+    auto scan = [&](uint32_t cnt, uint32_t& first, uint32_t& total) {
+        const uint32_t inc = wave_scan_incl_dpp(cnt);
+        first = inc - cnt;
+        total = __builtin_amdgcn_readlane(inc, 63);
+    };
+    auto escapes = [&](const uint2* t, uint32_t w, const uint32_t (&c)[2]) {
+        uint32_t n = 0;
+#pragma unroll
+        for (int g = 0; g < 4; ++g) n += add_escapes(group(t, w, c, g), ~3u);
+        return n;
+    };
+    // the four groups' bytes, completed by those `next` gives from a rank on
+    // (the entries looked up again: kept over the tiers below, they spill)
+    auto resolve = [&](const uint2* t, uint32_t w, const uint32_t (&c)[2], uint32_t q, auto next, uint32_t (&v)[4]) {
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            const uint2 en = group(t, w, c, g);
+            v[g] = complete(en, next(q));
+            q += add_escapes(en, ~3u);
+        }
+    };
+    const uint32_t ex_at = lds_address(ex);
+    auto terminal = [&](uint32_t q) {  // (read only where the directory gives the block words for it)
+        if (len <= pos) return 0u;
+        const u32x2 v = words(4 * pos + (q & ~3u));
+        return rotate_bytes(window_bytes(make_uint2(v.x, v.y), q));
+    };
+    auto below = [&](uint32_t q) { return window_bytes(lds_window(ex_at + q), q); };  // (ex_at is a whole word's)
+    auto put = [&](const uint32_t (&v)[4]) {
+#pragma unroll
+        for (int g = 0; g < 4; ++g) ex[4 * lane + g] = v[g];
+        wave_lds_sync();
+    };
+    constexpr uint32_t w0 = wave_width(P, 0), w1 = wave_width(P, 1);
+    uint32_t t0[2], q0, n1;
+    load(z.lit, z.n, w0, t0);
+    if constexpr (P == kWaveSip) {
+        keep(z.n, w0, t0);
+        scan(escapes(tab, w0, t0), q0, n1);
+        resolve(tab, w0, t0, q0, terminal, E);
+    } else {
+        uint32_t t1[2], q1, n2, v[4];
+        load(pos, 1024, w1, t1);
+        keep(z.n, w0, t0);
+        scan(escapes(tab, w0, t0), q0, n1);
+        pos += words_for(n1, w1);
+        keep(n1, w1, t1);
+        scan(escapes(tab + 256, w1, t1), q1, n2);
+        if constexpr (P == kWaveBalanced) {
+            resolve(tab + 256, w1, t1, q1, terminal, v);
+        } else {
+            uint32_t t2[2], q2, n3, cnt = 0;
+            load(pos, n2, 4, t2);
+            keep(n2, 4, t2);
+            auto pair = [&](int i) { return tab[512 + ((t2[i / 4] >> (8 * (i & 3))) & 0xFFu)]; };
+#pragma unroll
+            for (int i = 0; i < 8; ++i) cnt += add_escapes(pair(i), ~0u);
+            scan(cnt, q2, n3);
+            pos += words_for(n2, 4);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const uint2 en = pair(i);
+                const uint32_t two = (n3 ? complete(en, terminal(q2)) : en.x) & 0xFFFFu;
+                q2 += add_escapes(en, ~0u);
+                v[i / 2] = i & 1 ? v[i / 2] | two << 16 : two;
+            }
+            put(v);
+            resolve(tab + 256, w1, t1, q1, below, v);
+            wave_lds_sync();
+        }
+        put(v);
+        resolve(tab, w0, t0, q0, below, E);
+        wave_lds_sync();
+    }
+}
+
 // Decodes R blocks of size z (R = 2: a unit's rows; 1) from their loaded
 // stages: hi[j][g], lo[j][g] = the high and low bytes of the bf16 bits of the
 // lane's weights 4g .. 4g + 3 of block j (weight k in byte k). Weights past
@@ -282,19 +362,18 @@ __device__ __forceinline__ uint32_t complete(uint2 e, uint32_t next) { return __
 // compiler waits for each before it issues the next.
 template <int P, int R>
 __device__ __forceinline__ void wave_decode(const uint2* tab, uint32_t* ex, const WaveStage (&s)[R], const uint32_t* data,
-                                            const uint8_t* pal, const uint32_t (&start)[R], const int32_t (&len)[R],
-                                            const BlockSize& z, uint32_t lane, uint32_t (&hi)[R][4],
-                                            uint32_t (&lo)[R][4]) {
+                                            const uint32_t (&start)[R], const int32_t (&len)[R], const BlockSize& z,
+                                            uint32_t lane, uint32_t (&hi)[R][4], uint32_t (&lo)[R][4]) {
     constexpr uint32_t stride = wave_exchange(P);
     const uint32_t ex_at = lds_address(ex);
     uint2 e[R][4];
     uint32_t c[R][4];  // escapes of groups 0 .. g, less 4 (3 - g)
-    int32_t tail[R], bad = 0;  // (bad: negative once a limit is passed; every quantity is far below 2^31)
+    int32_t tail[R], bad[R];  // (bad: negative once a limit is passed; every quantity is far below 2^31)
     uint32_t T[R][2];
 #pragma unroll
     for (int j = 0; j < R; ++j) {
         tail[j] = len[j] - (int32_t)z.fixed;
-        bad |= 64 - tail[j];
+        bad[j] = 64 - tail[j];
         ex[j * stride + kExTerm + lane] = rotate_bytes(s[j].tail);
         if constexpr (P != kWaveSip) ex[j * stride + kExTail + lane] = s[j].tail;
         if constexpr (P == kWaveSip) {
@@ -351,7 +430,7 @@ __device__ __forceinline__ void wave_decode(const uint2* tab, uint32_t* ex, cons
     uint32_t below = kExTerm;  // where tier 0's escapes lie, in words of the exchange
     if constexpr (P == kWaveSip) {
 #pragma unroll
-        for (int j = 0; j < R; ++j) bad |= 4 * tail[j] - (int32_t)n1[j];
+        for (int j = 0; j < R; ++j) bad[j] |= 4 * tail[j] - (int32_t)n1[j];
     } else {
         // lane l: the block's tier-1 codes 8l .. 8l + 7
         constexpr uint32_t w = wave_width(P, 1);
@@ -401,7 +480,7 @@ __device__ __forceinline__ void wave_decode(const uint2* tab, uint32_t* ex, cons
 #pragma unroll
             for (int j = 0; j < R; ++j) {
                 const int32_t left = tail[j] - (int32_t)w1[j];  // terminal words
-                bad |= (512 - (int32_t)n1[j]) | left | (4 * left - (int32_t)n2[j]);
+                bad[j] |= (512 - (int32_t)n1[j]) | left | (4 * left - (int32_t)n2[j]);
                 windows(j, ex_at + 4 * (j * stride + kExTerm + (w1[j] & 63u)));
             }
         } else {
@@ -413,7 +492,7 @@ __device__ __forceinline__ void wave_decode(const uint2* tab, uint32_t* ex, cons
                 w2[j] = words_for(n2[j], 4);
                 const uint32_t code = reinterpret_cast<const uint8_t*>(ex + j * stride + kExTail + (w1[j] & 63u))[lane];
                 b[j] = tab[512 + keep_bits(code, (int32_t)(4 * n2[j]) - (int32_t)(8 * lane), 8)];
-                bad |= (512 - (int32_t)n1[j]) | (128 - (int32_t)n2[j]) | (tail[j] - (int32_t)(w1[j] + w2[j]));
+                bad[j] |= (512 - (int32_t)n1[j]) | (128 - (int32_t)n2[j]) | (tail[j] - (int32_t)(w1[j] + w2[j]));
             }
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -423,7 +502,7 @@ __device__ __forceinline__ void wave_decode(const uint2* tab, uint32_t* ex, cons
                 scan(cnt, q2, n3);
 #pragma unroll
                 for (int j = 0; j < R; ++j) {
-                    bad |= 4 * (tail[j] - (int32_t)(w1[j] + w2[j])) - (int32_t)n3[j];
+                    bad[j] |= 4 * (tail[j] - (int32_t)(w1[j] + w2[j])) - (int32_t)n3[j];
                     const uint32_t at = ex_at + 4 * (j * stride + kExTerm + ((w1[j] + w2[j]) & 63u)) + q2[j];
                     b[j].x = complete(b[j], window_bytes(lds_window(at), at));
                 }
@@ -458,12 +537,13 @@ __device__ __forceinline__ void wave_decode(const uint2* tab, uint32_t* ex, cons
         for (int g = 1; g < 4; ++g) E[j][g] = complete(e[j][g], window_bytes(win[j][g], c[j][g - 1]));
     }
     wave_lds_sync();
-    if (__builtin_expect(bad < 0, 0)) {
+    if (__builtin_expect((bad[0] | bad[R - 1]) < 0, 0)) {
 #pragma unroll 1
         for (int j = 0; j < R; ++j) {
+            if ((j ? bad[R - 1] : bad[0]) >= 0) continue;
             uint32_t x[4];
             const uint32_t at = j ? start[R - 1] : start[0];
-            wave_exact<P>(data, pal, at, at + (uint32_t)(j ? len[R - 1] : len[0]), z.n, lane, x);
+            wave_wide<P>(tab, ex, data, at, at + (uint32_t)(j ? len[R - 1] : len[0]), z, lane, x);
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
                 E[0][g] = j == 0 ? x[g] : E[0][g];
@@ -582,6 +662,8 @@ constexpr size_t wave_lds(int P, uint32_t W) {
 }
 static_assert(wave_exchange(kWaveSip) % 2 == 0 && wave_exchange(kWaveBalanced) % 2 == 0 && wave_exchange(kWaveGulp) % 2 == 0,
               "the exchanges are whole uint2");
+static_assert(wave_exchange(kWaveBalanced) >= 258 && wave_exchange(kWaveGulp) >= 258,
+              "wave_wide keeps 1024 exponent bytes and a window's overhang in an exchange");
 
 template <int P, int M, int XT>
 __global__ __launch_bounds__(wave_waves(P, M, XT) * 64, wave_occ(P, M, XT))
@@ -701,8 +783,7 @@ void k_gemv_wave(const WaveGroup g, const void* __restrict__ x, const WaveShape 
         float v[2 * M];
         uint32_t hi2[2][4], lo2[2][4];
         if constexpr (P != kWaveRaw)
-            wave_decode<P, 2>(tab, ex0, t.s, data, reinterpret_cast<const uint8_t*>(palette), t.start, t.len, size_of(cb),
-                              lane, hi2, lo2);
+            wave_decode<P, 2>(tab, ex0, t.s, data, t.start, t.len, size_of(cb), lane, hi2, lo2);
 #pragma unroll
         for (uint32_t j = 0; j < 2; ++j) {
             uint32_t wp[8];
@@ -844,7 +925,7 @@ __global__ __launch_bounds__(kDecodeWaves * 64, 4) void k_decode_wave(Desc d, ui
         const WaveStage st[1] = {s};
         const uint32_t start[1] = {(uint32_t)__builtin_amdgcn_readlane(o_start, k)};
         const int32_t len[1] = {(int32_t)(__builtin_amdgcn_readlane(o_end, k) - start[0])};
-        wave_decode<P, 1>(tab, ex, st, d.data, d.table, start, len, z, lane, hi, lo);
+        wave_decode<P, 1>(tab, ex, st, d.data, start, len, z, lane, hi, lo);
         wave_pairs(hi[0], lo[0], wp);
         uint16_t* dst = out + (uint64_t)row * d.cols + c * 1024 + 16 * lane;
         if (wide && 16 * lane + 16 <= w) {

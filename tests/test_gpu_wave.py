@@ -6,7 +6,8 @@ row counts (a unit's second row missing), a last block of 1, 4 and 1023
 weights, columns that are not dword-aligned, one block a row, more units than
 one directory read (32) a wave; and at escape densities from none to past
 every limit of the in-register tiers (512 tier-0 and 128 tier-1 escapes, 64
-tail words), which take the reads from memory."""
+tail words), which take the reads from memory; and at each such limit, one past
+it, and with every weight escaping as far as each tier."""
 
 import zlib
 
@@ -137,3 +138,101 @@ def test_gulp_rows_at_the_edge_of_the_wave_kernels_sums(cuda, M, blocks):
             w.copy_(bf16_tensor(bits, cuda))
             twin = dict(swap.to_device_twin(w, widths=rt["widths"], device=cuda), weight=w)
             assert torch.equal(radix_ops.gemv_rows(twin, x, None, torch.float32), y), start
+
+
+# (escapes of tier 0, of tier 1, of tier 2) of a block, by profile: none, the in-register tiers' limits (sip 256
+# terminal bytes; 512 and 128 escapes; 64 tail words) and one past each, every weight escaping as far as each tier
+COUNTS = {
+    "sip": [(0,), (1,), (255,), (256,), (257,), (700,), (1024,)],
+    "balanced": [(0, 0), (512, 60), (512, 64), (512, 65), (513, 0), (170, 180 - 12), (600, 600), (1024, 0),
+                 (1024, 1024), (1024, 1)],
+    "gulp": [(0, 0, 0), (512, 128, 64), (512, 128, 65), (512, 129, 0), (513, 0, 0), (512, 0, 0), (128, 128, 128),
+             (700, 300, 40), (1024, 0, 0), (1024, 1024, 0), (1024, 1024, 1024), (1024, 1, 1), (129, 129, 129)],
+}
+TIERS = {"sip": (7,), "balanced": (3, 7), "gulp": (3, 3, 15)}
+
+
+def _counted_bits(rng, profile, cols):
+    """Rows whose every 1024-weight block has the escape counts of one entry
+    of COUNTS (each next to each: a unit with one such row, and with two),
+    then rows that fix the palette's order."""
+    sizes = (*TIERS[profile], 19)
+    start = np.cumsum((0, *sizes))
+    exps = [125 - np.arange(start[t], start[t + 1]) for t in range(len(sizes))]
+
+    def block(counts):
+        left = 1024
+        tier = np.empty(1024, np.int64)
+        for t, c in enumerate((*counts, 0)):
+            c = min(c, left)
+            tier[c:left], left = t, c
+        rng.shuffle(tier)
+        return np.concatenate([exps[t][rng.integers(0, sizes[t], 1024)][:, None] for t in range(len(sizes))],
+                              axis=1)[np.arange(1024), tier]
+
+    nb = -(-cols // 1024)
+    rows = [np.concatenate([block(c) for _ in range(nb)])[:cols] for c in COUNTS[profile] for _ in range(2)]
+    rows += [rows[i] for i in rng.permutation(len(rows))]
+    share = {1: (.94, .06), 2: (.75, .22, .03), 3: (.65, .26, .08, .01)}[len(sizes) - 1]
+    every = np.concatenate(exps)
+    p = np.concatenate([np.full(n, s / n) for n, s in zip(sizes, share)])
+    filler = rng.choice(every, size=(len(rows) * 12, cols), p=p)
+    e = np.concatenate([np.array(rows), filler]).astype(np.uint16)
+    return (e << 7) | rng.integers(0, 128, e.shape, dtype=np.uint16) | (rng.integers(0, 2, e.shape, dtype=np.uint16) << 15), exps
+
+
+@pytest.mark.parametrize("cols", [2048, 1024 + 1000])
+@pytest.mark.parametrize("profile", ["sip", "balanced", "gulp"])
+def test_blocks_at_and_past_the_limits_of_the_in_register_tiers(cuda, profile, cols):
+    import torch
+
+    from drinkme_amd import radix_ops, swap
+
+    rng = np.random.default_rng(zlib.crc32(repr((profile, cols)).encode()))
+    bits, exps = _counted_bits(rng, profile, cols)
+    p = O.pack(bits, profile, allow_raw=False)
+    at = 0
+    for tier in exps[:-1]:  # the tiers' exponents are those the counts were made for
+        assert set(p.palette.reshape(-1)[at:at + len(tier)]) == set(tier)
+        at += len(tier)
+    rt = swap.to_device_radix(pack_to_dict(p, profile), cuda)
+    print(f"case wave counts {profile} {cols}", flush=True)
+    assert np.array_equal(u16_of(radix_ops.decode_bits(rt)), bits)
+    xf = rng.standard_normal((8, cols)).astype(np.float32)
+    for dtype, M in ((torch.bfloat16, 1), (torch.bfloat16, 4), (torch.float32, 2), (torch.float32, 8)):
+        x = torch.from_numpy(xf[:M]).to(cuda).to(dtype)
+        ref, bound = O.gemv_f64(bits, x.float().cpu().numpy())
+        y = radix_ops.gemv_rows(rt, x, None, torch.float32).cpu().numpy().astype(np.float64)
+        assert np.all(np.abs(y - ref) <= bound), f"{dtype} M={M}"
+
+
+def test_rows_of_different_scale_stay_near_the_unscaled_time(cuda):
+    """One palette over rows whose scales differ by a lognormal of sigma 0.5
+    puts a fifth of gulp's units past the in-register limits. Measured 1.5
+    times the unscaled launch; 4.3 on the gulp kernel, 7.8 where such blocks
+    are read a field at a time. The bound, 3, stands between."""
+    import torch
+
+    from drinkme_amd import radix_ops, radix_pack, swap
+
+    R, C = 12288, 4096
+    gen = torch.Generator(device=cuda).manual_seed(7)
+    w = torch.randn(R, C, generator=gen, device=cuda) * 0.02
+    scale = torch.exp(0.5 * torch.randn(R, 1, generator=gen, device=cuda))
+    x = torch.randn(1, C, generator=gen, device=cuda).to(torch.bfloat16)
+    took = []
+    for weight in (w, w * scale):
+        bits = u16_of(weight.to(torch.bfloat16))
+        call = radix_ops.RowsLauncher(swap.to_device_radix(radix_pack.pack_array_radix(bits, "gulp"), cuda))
+        best = float("inf")
+        for _ in range(5):
+            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            call(x)
+            a.record()
+            for _ in range(50):
+                call(x)
+            b.record()
+            torch.cuda.synchronize()
+            best = min(best, a.elapsed_time(b))
+        took.append(best)
+    assert took[1] < 3 * took[0], took

@@ -18,6 +18,8 @@ HIPCC = "/opt/rocm/bin/hipcc"
 # fences a block's decode takes by profile (0 sip, 1 balanced, 2 gulp): after the tail words, after each
 # resolved tier's bytes, and before the words are written again
 FENCES = {0: 2, 1: 3, 2: 4}
+# and wave_wide's: in the writer of a level's bytes, and after each read of them
+WIDE = {0: 0, 1: 2, 2: 3}
 
 
 @pytest.fixture(scope="module")
@@ -61,7 +63,7 @@ def _syncs(functions, body):
 
 
 def test_every_exchange_is_fenced(functions):
-    decoders, gulp = 0, {}
+    decoders, gulp, wide = 0, {}, {}
     for name, body in functions.items():
         decode = re.match(r"_ZN12_GLOBAL__N_111wave_decodeILi(\d)ELi\dEEEv", name)
         kernel = re.match(r"_ZZ?N12_GLOBAL__N_1(11k_gemv_gulpI\w*?EEEv)", name)  # (with its lambdas)
@@ -72,6 +74,12 @@ def test_every_exchange_is_fenced(functions):
             count, bare = _syncs(functions, body)
             assert bare == 0, name
             gulp[kernel.group(1)] = gulp.get(kernel.group(1), 0) + count
+        through = re.match(r"_ZZ?N12_GLOBAL__N_19wave_wideILi(\d)EEEv", name)  # (with its lambdas)
+        if through:
+            count, bare = _syncs(functions, body)
+            assert bare == 0, name
+            wide[int(through.group(1))] = wide.get(int(through.group(1)), 0) + count
     assert decoders == 6
+    assert wide == WIDE, wide
     # around the read of the tier-2 bytes
     assert gulp and set(gulp.values()) == {2}, gulp
