@@ -2355,9 +2355,9 @@ bool wave_first(const dmx_radix_tensor* t, uint32_t m) {
 }
 
 // One launch of the wave kernel over n tensors of profile p and equal cols
-// (already checked; kWaveRaw: t->data is the raw weight). Returns 2, having
+// (already checked; raw: the twin, t->data the raw weight). Returns 2, having
 // launched nothing, when two rows' sums per column block do not fit the LDS.
-int launch_wave(int p, const dmx_radix_tensor* const* ts, uint32_t n, const void* x, int x_dtype, uint32_t m,
+int launch_wave(int p, bool raw, const dmx_radix_tensor* const* ts, uint32_t n, const void* x, int x_dtype, uint32_t m,
                 const void* const* bias, int bias_dtype, void* const* out, int out_dtype, hipStream_t stream, char* err,
                 size_t errn) {
     if (n < 1 || n > (uint32_t)kGroupMax || m < 1 || m > 8) return 2;
@@ -2372,8 +2372,8 @@ int launch_wave(int p, const dmx_radix_tensor* const* ts, uint32_t n, const void
     sh.wide = xt == kWaveX32 || (sh.cols % 2 == 0 && reinterpret_cast<uintptr_t>(x) % 4 == 0);
     uint32_t rows[kGroupMax];
     for (uint32_t i = 0; i < n; ++i) rows[i] = ts[i]->rows;
-    const uint32_t M = 1u << mi, W = wave_waves(p, (int)M, xt);
-    sh.tile = wave_tile(rows, n, sh.nb, M, W, (uint32_t)cu_count() * wave_occ(p, (int)M, xt) * 4u / W, wave_lds(p, W));
+    const uint32_t M = 1u << mi;
+    sh.tile = wave_plan(p, raw, xt, M, rows, n, sh.nb, (uint32_t)cu_count());
     if (sh.tile == 0) return 2;
     WaveGroup g;
     uint64_t wgs = 0;
@@ -2389,7 +2389,9 @@ int launch_wave(int p, const dmx_radix_tensor* const* ts, uint32_t n, const void
         if (i < n) wgs += (ts[i]->rows + sh.tile - 1) / sh.tile;
         if (wgs >= (1ull << 31)) return 2;
     }
-    hipLaunchKernelGGL(wave_kernel(p, mi, xt), dim3((uint32_t)wgs), dim3(W * 64), sh.tile * sh.nb * M * 4, stream, g, x, sh);
+    const int kind = raw ? (int)kWaveRaw : p;
+    hipLaunchKernelGGL(wave_kernel(kind, mi, xt), dim3((uint32_t)wgs), dim3(wave_waves(kind, (int)M, xt) * 64),
+                       sh.tile * sh.nb * M * 4, stream, g, x, sh);
     return launch_check(err, errn, "wave gemv launch");
 }
 
@@ -2415,7 +2417,7 @@ int gemv_one(const dmx_radix_tensor* t, const Desc& d, const void* x, int x_dtyp
     const int p = wave_takes(t);
     const bool first = wave_first(t, m);
     if (first) {
-        const int rc = launch_wave(p, &t, 1, x, x_dtype, m, &bias, bias_dtype, &out, out_dtype, s, err, errn);
+        const int rc = launch_wave(p, false, &t, 1, x, x_dtype, m, &bias, bias_dtype, &out, out_dtype, s, err, errn);
         if (rc != 2) return rc;
     }
     if (sip_eligible(t, x, x_dtype, m)) {
@@ -2427,7 +2429,7 @@ int gemv_one(const dmx_radix_tensor* t, const Desc& d, const void* x, int x_dtyp
         if (rc != 2) return rc;
     }
     if (p >= 0 && !first) {
-        const int rc = launch_wave(p, &t, 1, x, x_dtype, m, &bias, bias_dtype, &out, out_dtype, s, err, errn);
+        const int rc = launch_wave(p, false, &t, 1, x, x_dtype, m, &bias, bias_dtype, &out, out_dtype, s, err, errn);
         if (rc != 2) return rc;
     }
     switch (m) {
@@ -2583,7 +2585,7 @@ extern "C" int dmx_radix_gemv_group(const dmx_radix_tensor* const* tensors, uint
     }
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (wave >= 0) {
-        const int rc = launch_wave(wave, tensors, n, x, x_dtype, m, bias, bias_dtype, out, out_dtype, s, err, errn);
+        const int rc = launch_wave(wave, false, tensors, n, x, x_dtype, m, bias, bias_dtype, out, out_dtype, s, err, errn);
         if (rc != 2) return rc;
     }
     if (all_sip) {
@@ -2733,7 +2735,7 @@ extern "C" int dmx_radix_gemv_twin(const uint16_t* w, uint32_t rows, uint32_t co
     const dmx_radix_tensor* tp = &t;
     const bool first = wave_first(&t, m);
     if (first) {
-        const int rc = launch_wave(kWaveRaw, &tp, 1, x, x_dtype, m, &bias, bias_dtype, &out, out_dtype, s, err, errn);
+        const int rc = launch_wave(wave_takes(&t), true, &tp, 1, x, x_dtype, m, &bias, bias_dtype, &out, out_dtype, s, err, errn);
         if (rc != 2) return rc;
     }
     if (fast && (is_sip(&t) || is_gulp(&t))) {
@@ -2741,7 +2743,7 @@ extern "C" int dmx_radix_gemv_twin(const uint16_t* w, uint32_t rows, uint32_t co
         if (rc != 2) return rc;
     }
     if (wave_takes(&t) >= 0 && !first) {
-        const int rc = launch_wave(kWaveRaw, &tp, 1, x, x_dtype, m, &bias, bias_dtype, &out, out_dtype, s, err, errn);
+        const int rc = launch_wave(wave_takes(&t), true, &tp, 1, x, x_dtype, m, &bias, bias_dtype, &out, out_dtype, s, err, errn);
         if (rc != 2) return rc;
     }
     Desc d = {};

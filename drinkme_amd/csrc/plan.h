@@ -566,6 +566,66 @@ inline bool plan_gulp(SipShape& sh, const uint32_t* row0, uint32_t n, uint32_t m
     return true;
 }
 
+// ---- the wave kernel (wave_kernels.h)
+
+enum WaveProfile { kWaveSip = 0, kWaveBalanced = 1, kWaveGulp = 2, kWaveRaw = 3 };
+
+// Profile of a tensor's widths, or -1.
+inline int wave_profile(uint32_t n_widths, const uint32_t* w) {
+    if (n_widths == 2 && w[0] == 3 && w[1] == 8) return kWaveSip;
+    if (n_widths == 3 && w[0] == 2 && w[1] == 3 && w[2] == 8) return kWaveBalanced;
+    if (n_widths == 4 && w[0] == 2 && w[1] == 2 && w[2] == 4 && w[3] == 8) return kWaveGulp;
+    return -1;
+}
+
+constexpr uint32_t wave_tiers(int P) { return P == kWaveSip ? 1u : P == kWaveBalanced ? 2u : 3u; }  // nonterminal
+constexpr uint32_t wave_width(int P, uint32_t j) {
+    return P == kWaveSip ? 3u : j == 0 ? 2u : P == kWaveBalanced ? 3u : j == 1 ? 2u : 4u;
+}
+
+// The activation types of the wave kernel.
+constexpr int kWaveX16 = 0, kWaveX32 = 1;
+
+// Decode table entries: sip 4096 (four 3-bit codes); balanced 256 (four 2-bit
+// codes) then 4096; gulp 256, 256 (four 2-bit codes each) and 256 (two 4-bit
+// codes).
+constexpr uint32_t wave_entries(int P) {
+    return P == kWaveSip ? 4096u : P == kWaveBalanced ? 256u + 4096u : P == kWaveGulp ? 768u : 1u;
+}
+
+// A wave's LDS exchange, in words, per row of a unit: the tail words rotated
+// (read as terminal bytes) and, past one tier, as they are (read as codes),
+// each with one word more; the tier-1 exponent bytes (512 and a window's
+// overhang) and the tier-2 ones (128 and the overhang).
+constexpr uint32_t kExTerm = 0, kExTail = 66, kExT1 = 132, kExT2 = kExT1 + 130;
+// (in front of the exchanges, in uint2: a window's address before its offset
+// is up to 12 bytes short of it)
+constexpr uint32_t kExHead = 2;
+constexpr uint32_t wave_exchange(int P) {
+    return P == kWaveSip ? kExTail : P == kWaveBalanced ? kExT2 : P == kWaveGulp ? kExT2 + 34 : 0u;
+}
+
+// Waves per workgroup, and the waves per SIMD the registers are cut to: two
+// 8-wave workgroups a CU (128 registers a wave) where the decode and the
+// activations fit that, one 12-wave workgroup (168) where they do not, one
+// 8-wave workgroup (256) for fp32 activations at M = 8 (128 registers of
+// them).
+constexpr bool wave_one_wg(int P, int M, int XT) {
+    return P != kWaveRaw && M == (XT == kWaveX32 ? 4 : 8);
+}
+constexpr uint32_t wave_waves(int P, int M, int XT) { return wave_one_wg(P, M, XT) ? 12u : 8u; }
+constexpr uint32_t wave_occ(int P, int M, int XT) {
+    return wave_one_wg(P, M, XT) ? 3u : XT == kWaveX32 && M == 8 ? 2u : 4u;
+}
+// static LDS of the wave kernel
+constexpr size_t wave_lds(int P, uint32_t W) {
+    return 8 * (kExHead + (size_t)W * wave_exchange(P) + wave_entries(P));
+}
+static_assert(wave_exchange(kWaveSip) % 2 == 0 && wave_exchange(kWaveBalanced) % 2 == 0 && wave_exchange(kWaveGulp) % 2 == 0,
+              "the exchanges are whole uint2");
+static_assert(wave_exchange(kWaveBalanced) >= 258 && wave_exchange(kWaveGulp) >= 258,
+              "wave_wide keeps 1024 exponent bytes and a window's overhang in an exchange");
+
 // The wave kernel's rows per workgroup T (even) for n tensors of rows[i]
 // rows and nb column blocks: the T that takes the fewest unit times, a
 // workgroup's being its waves' longest run of units and kWaveSetup of them
@@ -600,6 +660,20 @@ inline uint32_t wave_tile(const uint32_t* rows, uint32_t n, uint32_t nb, uint32_
         }
     }
     return (uint32_t)best;
+}
+
+// The wave kernel's tile for tensors of profile p, or 0 where it does not take
+// them; raw: for the raw twin of such a tensor, which it takes exactly where
+// it takes the tensor (the two run the same kernel, so that their sums are the
+// same), though the raw kernel's own LDS would hold longer rows.
+inline uint32_t wave_plan(int p, bool raw, int xt, uint32_t M, const uint32_t* rows, uint32_t n, uint32_t nb,
+                          uint32_t cus) {
+    auto tile = [&](int P) {
+        const uint32_t W = wave_waves(P, (int)M, xt);
+        return wave_tile(rows, n, nb, M, W, cus * wave_occ(P, (int)M, xt) * 4u / W, wave_lds(P, W));
+    };
+    const uint32_t t = tile(p);
+    return raw && t ? tile(kWaveRaw) : t;
 }
 
 }  // namespace dmx

@@ -50,52 +50,6 @@
 // tier-0 or 128 tier-1 escapes, a tail of more than 64 words, streams cut
 // short) takes wave_wide, which reads its streams from memory.
 
-enum WaveProfile { kWaveSip = 0, kWaveBalanced = 1, kWaveGulp = 2, kWaveRaw = 3 };
-
-// Profile of a tensor's widths, or -1.
-inline int wave_profile(uint32_t n_widths, const uint32_t* w) {
-    if (n_widths == 2 && w[0] == 3 && w[1] == 8) return kWaveSip;
-    if (n_widths == 3 && w[0] == 2 && w[1] == 3 && w[2] == 8) return kWaveBalanced;
-    if (n_widths == 4 && w[0] == 2 && w[1] == 2 && w[2] == 4 && w[3] == 8) return kWaveGulp;
-    return -1;
-}
-
-constexpr uint32_t wave_tiers(int P) { return P == kWaveSip ? 1u : P == kWaveBalanced ? 2u : 3u; }  // nonterminal
-constexpr uint32_t wave_width(int P, uint32_t j) {
-    return P == kWaveSip ? 3u : j == 0 ? 2u : P == kWaveBalanced ? 3u : j == 1 ? 2u : 4u;
-}
-// byte offset of tier j's run in the padded palette tables
-constexpr uint32_t wave_pal_byte(int P, uint32_t j) {
-    uint32_t b = 0;
-    for (uint32_t k = 0; k < j; ++k) b += 1u << wave_width(P, k);
-    return b;
-}
-
-// The activation types of the wave kernel, its element reads and stores.
-constexpr int kWaveX16 = 0, kWaveX32 = 1;
-
-struct WaveTables {
-    // entries of kWaveSip: 4096 (four 3-bit codes); balanced: 256 (four 2-bit
-    // codes) then 4096; gulp: 256, 256 (four 2-bit codes each) and 256 (two
-    // 4-bit codes)
-    static constexpr uint32_t entries(int P) {
-        return P == kWaveSip ? 4096u : P == kWaveBalanced ? 256u + 4096u : P == kWaveGulp ? 768u : 1u;
-    }
-    static constexpr uint32_t tier(int P, uint32_t j) { return j == 0 ? 0u : j == 1 ? 256u : 512u; }
-};
-
-// A wave's LDS exchange, in words, per row of a unit: the tail words rotated
-// (read as terminal bytes) and, past one tier, as they are (read as codes),
-// each with one word more; the tier-1 exponent bytes (512 and a window's
-// overhang) and the tier-2 ones (128 and the overhang).
-constexpr uint32_t kExTerm = 0, kExTail = 66, kExT1 = 132, kExT2 = kExT1 + 130;
-// (in front of the exchanges, in uint2: a window's address before its offset
-// is up to 12 bytes short of it)
-constexpr uint32_t kExHead = 2;
-constexpr uint32_t wave_exchange(int P) {
-    return P == kWaveSip ? kExTail : P == kWaveBalanced ? kExT2 : P == kWaveGulp ? kExT2 + 34 : 0u;
-}
-
 // Exponent bytes are kept rotated right by one: a byte's low seven bits are
 // the bf16 high byte's and its top bit the low byte's, so merging them with
 // the literals (sign and mantissa) takes one v_bfi a half.
@@ -643,34 +597,13 @@ struct __attribute__((packed, aligned(4))) Quad4 {
     uint32_t v[4];
 };
 
-// Waves per workgroup, and the waves per SIMD the registers are cut to: two
-// 8-wave workgroups a CU (128 registers a wave) where the decode and the
-// activations fit that, one 12-wave workgroup (168) where they do not, one
-// 8-wave workgroup (256) for fp32 activations at M = 8 (128 registers of
-// them).
-constexpr bool wave_wide(int P, int M, int XT) {
-    return P != kWaveRaw && M == (XT == kWaveX32 ? 4 : 8);
-}
-constexpr uint32_t wave_waves(int P, int M, int XT) { return wave_wide(P, M, XT) ? 12u : 8u; }
-constexpr uint32_t wave_occ(int P, int M, int XT) {
-    return wave_wide(P, M, XT) ? 3u : XT == kWaveX32 && M == 8 ? 2u : 4u;
-}
 constexpr uint32_t kDecodeWaves = 8;
-// static LDS of the wave kernel
-constexpr size_t wave_lds(int P, uint32_t W) {
-    return 8 * (kExHead + (size_t)W * wave_exchange(P) + WaveTables::entries(P));
-}
-static_assert(wave_exchange(kWaveSip) % 2 == 0 && wave_exchange(kWaveBalanced) % 2 == 0 && wave_exchange(kWaveGulp) % 2 == 0,
-              "the exchanges are whole uint2");
-static_assert(wave_exchange(kWaveBalanced) >= 258 && wave_exchange(kWaveGulp) >= 258,
-              "wave_wide keeps 1024 exponent bytes and a window's overhang in an exchange");
-
 template <int P, int M, int XT>
 __global__ __launch_bounds__(wave_waves(P, M, XT) * 64, wave_occ(P, M, XT))
 void k_gemv_wave(const WaveGroup g, const void* __restrict__ x, const WaveShape sh) {
     constexpr uint32_t W = wave_waves(P, M, XT);
     constexpr int XR = XT == kWaveX32 ? 16 : 8;  // activation registers per row
-    __shared__ __align__(16) uint2 lds[kExHead + W * wave_exchange(P) + WaveTables::entries(P)];
+    __shared__ __align__(16) uint2 lds[kExHead + W * wave_exchange(P) + wave_entries(P)];
     uint2* tab = lds + kExHead + W * wave_exchange(P);
     extern __shared__ __align__(16) uint8_t lds_dyn[];
     float* red = reinterpret_cast<float*>(lds_dyn);
@@ -900,7 +833,7 @@ template <int P>
 __global__ __launch_bounds__(kDecodeWaves * 64, 4) void k_decode_wave(Desc d, uint16_t* __restrict__ out, uint32_t run,
                                                                      uint32_t wide) {
     constexpr uint32_t W = kDecodeWaves;
-    __shared__ __align__(16) uint2 lds[kExHead + W * wave_exchange(P) / 2 + WaveTables::entries(P)];
+    __shared__ __align__(16) uint2 lds[kExHead + W * wave_exchange(P) / 2 + wave_entries(P)];
     uint2* tab = lds + kExHead + W * wave_exchange(P) / 2;
     const uint32_t wv = wave_id(), lane = lane_id(), blocks = d.rows * d.nb;
     const uint32_t b0 = min(blocks, (blockIdx.x * W + wv) * run), n = min(run, blocks - b0);

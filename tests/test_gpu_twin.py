@@ -120,3 +120,24 @@ def test_twin_matches_on_a_launch_long_enough_for_progress_balance(cuda, profile
     ref, bound = O.gemv_f64(bits, O.bf16_bits_to_f32(xb[:1]))
     yy = y.cpu().numpy().astype(np.float64)
     assert np.all(np.abs(yy - ref.reshape(yy.shape)) <= bound.reshape(yy.shape))
+
+
+@pytest.mark.parametrize("dtype,M,blocks", [("bfloat16", 8, 86), ("bfloat16", 8, 87), ("bfloat16", 5, 90), ("float32", 3, 173),
+                                            ("float32", 4, 174), ("bfloat16", 8, 256)])
+def test_long_balanced_rows_and_their_twin_run_the_same_kernel(cuda, dtype, M, blocks):
+    """balanced's twelve-wave workgroups (M = 8; fp32, M = 4) keep the sums of
+    86 and 173 column blocks beside their tables. The raw kernel has room for
+    more: the twin leaves the wave kernel where its tensor does."""
+    import torch
+
+    from drinkme_amd import radix_ops
+
+    rng = np.random.default_rng(blocks + M)
+    bits = escape_heavy_bits(rng, (3, 1024 * blocks), 0.03)
+    p, twin = _pair(bits, "balanced", cuda)
+    x = torch.from_numpy(rng.standard_normal((M, 1024 * blocks)).astype(np.float32)).to(cuda).to(getattr(torch, dtype))
+    print(f"case twin long balanced {dtype} M={M} blocks={blocks}", flush=True)
+    y = radix_ops.gemv_mc(p, x)
+    assert torch.equal(radix_ops.gemv_mc(twin, x), y)
+    ref, bound = O.gemv_f64(bits, x.float().cpu().numpy())
+    assert np.all(np.abs(y.cpu().numpy().astype(np.float64) - ref) <= bound)

@@ -13,8 +13,9 @@ past its work as far as a load pipeline runs ahead. It also decodes every
 code pattern through the gulp tables as the kernel looks them up (the
 tables' entries and lookup are plan.h's, shared with the kernel) against a
 direct decode: a layout mistake there only sends blocks down the exact
-fallback, correct but slow, so no parity test would see it. The five planted
-mistakes are its negative controls: each must be caught."""
+fallback, correct but slow, so no parity test would see it. And it plans the
+wave kernel's launches: a raw twin is taken exactly where its compressed tensor
+is. The six planted mistakes are its negative controls: each must be caught."""
 
 import os
 import subprocess
@@ -42,7 +43,7 @@ def test_every_walk_stays_in_range_and_covers_each_block_once(model):
     assert plans > 500
 
 
-@pytest.mark.parametrize("plant", [1, 2, 3, 4, 5])
+@pytest.mark.parametrize("plant", [1, 2, 3, 4, 5, 6])
 def test_planted_walk_mistakes_are_caught(model, plant):
     res = subprocess.run([model, "--plant", str(plant)], capture_output=True, text=True, timeout=300)
     assert res.returncode == 0 and "caught" in res.stdout and "NOT" not in res.stdout, res.stdout + res.stderr

@@ -17,7 +17,7 @@
 // It also checks the per-lane load offsets against the reach pad.
 //
 //   walk_model            every configuration; exit status 0 when clean
-//   walk_model --plant K  the same with planted mistake K (1..4) in the
+//   walk_model --plant K  the same with planted mistake K (1..6) in the
 //                         walk it models; exit status 0 when the checks
 //                         catch it (a negative control)
 #include <stdint.h>
@@ -330,11 +330,41 @@ void check_gulp_tables() {
     }
 }
 
+// The wave kernel takes a raw twin exactly where it takes the compressed
+// tensor of its profile (both then run it, or neither), and what it takes
+// fits its LDS: every profile, activation type, row count and column block
+// count up to past the longest rows that it takes, at groups and CU counts of
+// several sizes. (Planted mistake 6: the twin by the raw kernel's own LDS.)
+void check_wave_plans() {
+    const std::vector<std::vector<uint32_t>> groups = {{1}, {3}, {4096}, {12288, 12288}, {6144, 1, 1024, 17}};
+    for (int p : {kWaveSip, kWaveBalanced, kWaveGulp})
+        for (int xt : {kWaveX16, kWaveX32})
+            for (uint32_t M : {1u, 2u, 4u, 8u})
+                for (uint32_t nb = 1; nb <= 2100; ++nb)
+                    for (const auto& rows : groups)
+                        for (uint32_t cus : {256u, 7u}) {
+                            const uint32_t n = (uint32_t)rows.size();
+                            const uint32_t t = wave_plan(p, false, xt, M, rows.data(), n, nb, cus);
+                            const uint32_t r = wave_plan(g_plant == 6 ? (int)kWaveRaw : p, true, xt, M, rows.data(), n, nb, cus);
+                            const std::string what = "wave plan: profile " + std::to_string(p) + " xt " + std::to_string(xt) +
+                                                     " M " + std::to_string(M) + " nb " + std::to_string(nb);
+                            if ((t == 0) != (r == 0)) bad(what + ": the twin's kernel is another");
+                            for (int raw : {0, 1}) {
+                                const uint32_t tile = raw ? r : t;
+                                const int kind = raw ? (int)kWaveRaw : p;
+                                if (tile % 2) bad(what + ": an odd tile");
+                                if (tile && (size_t)tile * nb * M * 4 + wave_lds(kind, wave_waves(kind, (int)M, xt)) > 64 * 1024)
+                                    bad(what + ": past 64 KB of LDS");
+                            }
+                        }
+}
+
 int main(int argc, char** argv) {
     if (argc == 3 && !strcmp(argv[1], "--plant")) g_plant = atoi(argv[2]);
     check_reach();
     check_gulp_t1();
     check_gulp_tables();
+    check_wave_plans();
     // the configurations' launches: Qwen3-8B (q/k/v, o, gate/up, down,
     // lm_head) and the 32B class, grouped as the benchmark groups them
     const std::vector<std::pair<std::vector<uint32_t>, uint32_t>> shapes = {
