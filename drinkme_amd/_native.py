@@ -11,6 +11,7 @@ import ctypes as ct
 import importlib.machinery
 import importlib.util
 import os
+import warnings
 
 from .build import CALLS, LIB
 
@@ -100,23 +101,37 @@ def lib():
     return _lib
 
 
-_calls = None
+_UNLOADED = object()
+_calls = _UNLOADED
+
+
+def _load_calls():
+    import torch  # (the extension links torch's libraries, which this loads)
+
+    lib()
+    if not os.path.exists(CALLS):
+        raise ImportError(f"{CALLS} is not built; run `python -m drinkme_amd.build`")
+    loader = importlib.machinery.ExtensionFileLoader("dmx_calls", CALLS)
+    module = importlib.util.module_from_spec(importlib.util.spec_from_loader("dmx_calls", loader))
+    loader.exec_module(module)
+    if module.torch_version != torch.__version__:  # (tensors are passed by torch's own C++ layouts)
+        raise ImportError(f"{CALLS} was built for torch {module.torch_version}, this is {torch.__version__}")
+    return module
 
 
 def calls():
     """The loaded extension of the launchers' per-call path
-    (csrc/torch_calls.cpp; raises when it is not built)."""
+    (csrc/torch_calls.cpp), or None, with one warning, where it is not built
+    or not for this torch: the launchers then launch the same kernels through
+    the C ABI, at more host time a call."""
     global _calls
-    if _calls is None:
-        import torch  # noqa: F401  (the extension links torch's libraries, which this loads)
-
-        lib()
-        if not os.path.exists(CALLS):
-            raise ImportError(f"dmx_calls.so is not built ({CALLS}); run `python -m drinkme_amd.build`")
-        loader = importlib.machinery.ExtensionFileLoader("dmx_calls", CALLS)
-        module = importlib.util.module_from_spec(importlib.util.spec_from_loader("dmx_calls", loader))
-        loader.exec_module(module)
-        _calls = module
+    if _calls is _UNLOADED:
+        try:
+            _calls = _load_calls()
+        except ImportError as e:
+            warnings.warn(f"drinkme_amd: launches go through ctypes (slower on the host): {e}", RuntimeWarning,
+                          stacklevel=3)
+            _calls = None
     return _calls
 
 

@@ -79,7 +79,8 @@ def build(verbose: bool = False) -> str:
     dirs = [os.path.join(home, "include"), os.path.join(home, "include", "torch", "csrc", "api", "include"),
             sysconfig.get_paths()["include"]]
     _run([*host, "-O2", *(f for d in dirs for f in ("-isystem", d)),
-          f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-shared",
+          f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+          f'-DDMX_TORCH_VERSION="{torch.__version__}"', "-shared",
           os.path.join(CSRC, "torch_calls.cpp"), "-L" + LIBDIR, "-l:" + os.path.basename(LIB),
           "-L" + os.path.join(home, "lib"), "-ltorch_python", "-ltorch_cpu", "-lc10", "-Wl,-rpath,$ORIGIN",
           "-o", CALLS + ".tmp"], verbose)

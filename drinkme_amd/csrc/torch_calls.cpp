@@ -216,5 +216,11 @@ PyMODINIT_FUNC PyInit_dmx_calls(void) {
     const char* names[4] = {"rx_data", "rx_offsets", "rx_palette", "rx_schedule"};
     for (int i = 0; i < 4; ++i)
         if (!(g_keys[i] = PyUnicode_InternFromString(names[i]))) return nullptr;
-    return PyModule_Create(&g_module);
+    PyObject* m = PyModule_Create(&g_module);
+    // (the torch whose headers this was compiled with: the loader compares)
+    if (m && PyModule_AddStringConstant(m, "torch_version", DMX_TORCH_VERSION) < 0) {
+        Py_DECREF(m);
+        return nullptr;
+    }
+    return m;
 }

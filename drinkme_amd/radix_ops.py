@@ -243,9 +243,9 @@ class RowsLauncher:
 
     def __call__(self, x: torch.Tensor, bias=None, out_dtype=torch.float32) -> torch.Tensor:
         live = self._live  # (held through the call: another thread may rebuild the descriptor meanwhile)
-        if live is not None:  # the plain case in one native call; None: anything else
-            out = _native.calls().rows(live[1], self.p, x, bias, out_dtype, self.R, self.C, self._dev,
-                                       _stream(self.device))
+        native = _native.calls() if live is not None else None
+        if native is not None:  # the plain case in one native call; None: anything else
+            out = native.rows(live[1], self.p, x, bias, out_dtype, self.R, self.C, self._dev, _stream(self.device))
             if out is not None:
                 return out
         M = _leading_rows(x, self.C, self.device, "radix gemv")
@@ -282,7 +282,8 @@ def gemv_narrow(w: torch.Tensor, x: torch.Tensor, bias, block: int = 512, num_wa
 def narrow_rows(w: torch.Tensor, x: torch.Tensor, bias):
     """gemv_narrow for x [..., C] -> [..., R] in one native call, or None
     (nothing launched) where it does not take these tensors as they are."""
-    return _native.calls().narrow(w, x, bias, _stream(x.device))
+    native = _native.calls()
+    return native.narrow(w, x, bias, _stream(x.device)) if native is not None else None
 
 
 def gemv_fused(p: dict, x: torch.Tensor, bias, out_dtype=torch.bfloat16) -> torch.Tensor:
@@ -380,9 +381,10 @@ class GroupLauncher:
         if biases is not None and any(b is not None for b in biases):
             bias_arr, bd, biases = self._bias_array(biases, x)  # (the contiguous biases live through the call)
         live = self._live  # (held through the call, as in RowsLauncher)
-        if live is not None:
-            outs = _native.calls().group(live[2], self.ps, x, ct.addressof(bias_arr) if bias_arr is not None else 0,
-                                         bd, out_dtype, live[3], self.C, self._dev, _stream(self.device))
+        native = _native.calls() if live is not None else None
+        if native is not None:
+            outs = native.group(live[2], self.ps, x, ct.addressof(bias_arr) if bias_arr is not None else 0, bd,
+                                out_dtype, live[3], self.C, self._dev, _stream(self.device))
             if outs is not None:
                 return outs
         tarr = self._table()

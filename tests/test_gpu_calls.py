@@ -113,3 +113,24 @@ def test_narrow_equals_the_general_path(cuda):
         with torch.no_grad():
             x9 = torch.randn(9, C, device=cuda, dtype=torch.bfloat16)
             assert torch.equal(mod(x9), torch.nn.functional.linear(x9, lin.weight, b))
+
+
+def test_without_the_extension_the_general_path_gives_the_same(cuda, monkeypatch):
+    import torch
+
+    from drinkme_amd import _native, radix_ops, swap
+
+    p, = _tensors(cuda, (257,))
+    one, many = radix_ops.RowsLauncher(p), radix_ops.GroupLauncher([p, p])
+    lin = torch.nn.Linear(C, 48, bias=True, device=cuda, dtype=torch.bfloat16)
+    mod = swap.NarrowLinear.adopt(lin)
+    x = torch.randn(3, C, device=cuda).to(torch.bfloat16)
+    with torch.no_grad():
+        def passes():
+            return [one(x), *many(x), mod(x)]
+
+        passes()  # (builds the descriptors)
+        want = passes()
+        monkeypatch.setattr(_native, "_calls", None)
+        for got, y in zip(passes(), want):
+            assert got.shape == y.shape and torch.equal(got, y)
