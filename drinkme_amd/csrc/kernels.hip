@@ -1409,14 +1409,13 @@ __device__ __forceinline__ void gulp_tables(uint4* t0tab, uint2* t1tab, uint8_t*
 
 // DEC: decode only, each block's bf16 bits stored to the tensor's output
 // (row-major [rows, cols]) in place of the products.
-// WV: waves per workgroup, the plan's (12, or 8 at three workgroups per CU).
 // MX: the matrix policy (M = 4 in quad units, as M = 8).
-template <int M, bool PH, bool DEC = false, int WV = kSipWaves, bool MX = false>
-__global__ __launch_bounds__(WV * 64, (M == 8 || (M == 4 && gulp_quad(4, MX))) ? 3 : 6)
+template <int M, bool PH, bool DEC = false, bool MX = false>
+__global__ __launch_bounds__(kSipThreads, (M == 8 || (M == 4 && gulp_quad(4, MX))) ? 3 : 6)
 void k_gemv_gulp(const SipGroup g, const uint16_t* __restrict__ x, const SipShape sh) {
     static_assert(!DEC || (M == 1 && !PH), "the decode runs unphased");
-    static_assert(WV == kSipWaves || (!PH && !DEC && !gulp_quad(M, MX)), "8-wave workgroups run unphased v_dot2 rows");
-    constexpr uint32_t W = WV, TH = 64u * WV;
+    static_assert(PH || DEC || gulp_quad(M, MX), "v_dot2 rows of one phase are the wave kernel's");
+    constexpr uint32_t W = kSipWaves, TH = kSipThreads;
     // verify rows four output rows at a time on the matrix cores
     constexpr bool QUAD = !DEC && gulp_quad(M, MX);
     __shared__ uint4 t0tab[256];
@@ -2240,19 +2239,16 @@ bool gulp_eligible(const dmx_radix_tensor* t, const void* x, int x_dtype, uint32
 
 typedef void (*GulpKernel)(const SipGroup, const uint16_t*, const SipShape);
 
-// waves: the plan's waves per workgroup (8 only unphased, M <= 4);
-// matrix: the matrix policy's M = 4 (quad units)
-GulpKernel gulp_kernel(bool phased, int mi, uint32_t waves = kSipWaves, bool matrix = false) {
+// k_gemv_gulp for M = 1, 2, 4, 8 (mi 0..3), one column phase or several;
+// matrix: the matrix policy's M = 4 (quad units). Null: M <= 4 in one phase,
+// which the wave kernel takes (its rows end at 2048 / M column blocks, 4 MB of
+// activations, long past what one phase holds).
+GulpKernel gulp_kernel(bool phased, int mi, bool matrix) {
     static const GulpKernel table[2][4] = {
-        {k_gemv_gulp<1, false>, k_gemv_gulp<2, false>, k_gemv_gulp<4, false>, k_gemv_gulp<8, false>},
+        {nullptr, nullptr, nullptr, k_gemv_gulp<8, false>},
         {k_gemv_gulp<1, true>, k_gemv_gulp<2, true>, k_gemv_gulp<4, true>, k_gemv_gulp<8, true>}};
-    static const GulpKernel table8[3] = {k_gemv_gulp<1, false, false, kGulpWaves3>,
-                                         k_gemv_gulp<2, false, false, kGulpWaves3>,
-                                         k_gemv_gulp<4, false, false, kGulpWaves3>};
-    static const GulpKernel matrix4[2] = {k_gemv_gulp<4, false, false, kSipWaves, true>,
-                                          k_gemv_gulp<4, true, false, kSipWaves, true>};
-    if (matrix && mi == 2) return matrix4[phased ? 1 : 0];
-    return waves == kGulpWaves3 && !phased && mi < 3 ? table8[mi] : table[phased ? 1 : 0][mi];
+    static const GulpKernel matrix4[2] = {k_gemv_gulp<4, false, false, true>, k_gemv_gulp<4, true, false, true>};
+    return matrix && mi == 2 ? matrix4[phased ? 1 : 0] : table[phased ? 1 : 0][mi];
 }
 
 // One launch of the gulp kernel over n tensors of equal cols (already
@@ -2298,16 +2294,16 @@ int launch_gulp(const dmx_radix_tensor* const* ts, uint32_t n, const void* x, ui
     bool two = false;
     const bool matrix = matrix_policy() && mi == 2;
     if (!plan_gulp(sh, g.row0, n, min_rows, M, (uint32_t)cu_count(), grid, lds, two, matrix)) return 2;
+    const GulpKernel kern = gulp_kernel(sh.phases > 1, mi, matrix);
+    if (!kern) return 2;
     {
-        const void* kerns[13];
-        for (int t = 0; t < 2; ++t)
-            for (int i = 0; i < 4; ++i) kerns[4 * t + i] = reinterpret_cast<const void*>(gulp_kernel(t, i));
-        for (int i = 0; i < 3; ++i) kerns[8 + i] = reinterpret_cast<const void*>(gulp_kernel(false, i, kGulpWaves3));
-        for (int t = 0; t < 2; ++t) kerns[11 + t] = reinterpret_cast<const void*>(gulp_kernel(t, 2, kSipWaves, true));
-        if (raise_lds_limit(kFamGulp, kerns, 13, lds, 64 * 1024 - fixed, "gulp kernel LDS opt-in", err, errn)) return 1;
+        const void* kerns[7];
+        for (int i = 0; i < 4; ++i) kerns[i] = reinterpret_cast<const void*>(gulp_kernel(true, i, false));
+        kerns[4] = reinterpret_cast<const void*>(gulp_kernel(false, 3, false));
+        for (int t = 0; t < 2; ++t) kerns[5 + t] = reinterpret_cast<const void*>(gulp_kernel(t, 2, true));
+        if (raise_lds_limit(kFamGulp, kerns, 7, lds, 64 * 1024 - fixed, "gulp kernel LDS opt-in", err, errn)) return 1;
     }
-    if (sh.waves != kSipWaves && (sh.waves != kGulpWaves3 || sh.phases > 1 || mi == 3 || matrix)) return 2;
-    hipLaunchKernelGGL(gulp_kernel(sh.phases > 1, mi, sh.waves, matrix), dim3(grid), dim3(64u * sh.waves), lds, stream,
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(kSipThreads), lds, stream,
                        g, static_cast<const uint16_t*>(x), sh);
     return launch_check(err, errn, "gulp gemv launch");
 }
@@ -2638,14 +2634,15 @@ typedef void (*RawKernel)(const SipGroup, const uint16_t*, const SipShape);
 
 // k_gemv_sip's raw instantiations: phased or not; M = 1, 2, 4, 8 (mi); at
 // M = 4 and 8 the verify-row rule of the kernel mirrored (sip: quad units on
-// the matrix cores; gulp: v_dot2 at M = 4, quad units with gulp's tiles at
-// M = 8). At M = 1 and 2 the sip and gulp kernels do the same arithmetic,
-// so one instantiation mirrors both.
+// the matrix cores; gulp: v_dot2 at M = 4, in several phases only, as
+// gulp_kernel says, quad units with gulp's tiles at M = 8). At M = 1 and 2 the
+// sip and gulp kernels do the same arithmetic, so one instantiation mirrors
+// both.
 constexpr int kRawKinds = 7;
 RawKernel raw_kernel(bool phased, int kind) {
     static const RawKernel table[2][kRawKinds] = {
         {k_gemv_sip<false, 1, false, 1>, k_gemv_sip<false, 2, false, 1>, k_gemv_sip<false, 4, false, 1>,
-         k_gemv_sip<false, 8, false, 1>, k_gemv_sip<false, 4, false, 2>, k_gemv_sip<false, 8, false, 2>,
+         k_gemv_sip<false, 8, false, 1>, nullptr, k_gemv_sip<false, 8, false, 2>,
          k_gemv_sip<false, 4, false, kModeTwinGulpMx>},
         {k_gemv_sip<false, 1, true, 1>, k_gemv_sip<false, 2, true, 1>, k_gemv_sip<false, 4, true, 1>,
          k_gemv_sip<false, 8, true, 1>, k_gemv_sip<false, 4, true, 2>, k_gemv_sip<false, 8, true, 2>,
@@ -2695,16 +2692,19 @@ int launch_raw(const uint16_t* w, uint32_t rows, uint32_t cols, bool gulp, const
                      fixed, !gulp, (uint32_t)cu_count(), grid, lds, two))
         return 2;
     if ((uint64_t)sh.rows_per_wg * cols * 2 >= (1ull << 31)) return 2;  // a tile's bytes within the buffer range
+    const RawKernel kern = raw_kernel(sh.phases > 1, raw_kind(mi, gulp, matrix));
+    if (!kern) return 2;
     {
         const void* kerns[2 * kRawKinds];  // (the raw kernels declare sip's static LDS)
+        int nk = 0;
         for (int t = 0; t < 2; ++t)
-            for (int i = 0; i < kRawKinds; ++i) kerns[kRawKinds * t + i] = reinterpret_cast<const void*>(raw_kernel(t, i));
-        if (raise_lds_limit(kFamRaw, kerns, 2 * kRawKinds, lds, 64 * 1024 - kSipStaticLds, "raw twin kernel LDS opt-in", err,
+            for (int i = 0; i < kRawKinds; ++i)
+                if (raw_kernel(t, i)) kerns[nk++] = reinterpret_cast<const void*>(raw_kernel(t, i));
+        if (raise_lds_limit(kFamRaw, kerns, nk, lds, 64 * 1024 - kSipStaticLds, "raw twin kernel LDS opt-in", err,
                             errn))
             return 1;
     }
-    hipLaunchKernelGGL(raw_kernel(sh.phases > 1, raw_kind(mi, gulp, matrix)), dim3(grid), dim3(kSipThreads), lds, stream,
-                       g, static_cast<const uint16_t*>(x), sh);
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(kSipThreads), lds, stream, g, static_cast<const uint16_t*>(x), sh);
     return launch_check(err, errn, "raw twin gemv launch");
 }
 

@@ -26,9 +26,10 @@ and padded model (:149-182) are restated here for this build's kernels:
     reaches more than 768 words past a block's start, and 16 + 4096 words
     follow the payload.
 
-Both the whole-block tensors the sip and gulp kernels take (M = 1, 4, 8:
-the v_dot2 and matrix-core paths) and a ragged tensor (two full blocks and
-a 52-weight tail per row, the generic kernel) are covered. The runtime
+Both whole-block tensors (M = 1, 4, 8: the sip and gulp kernels' v_dot2 and
+matrix-core paths, the wave kernel's for gulp at M <= 4 and for balanced) and a
+ragged tensor (two full blocks and a 52-weight tail per row, the wave kernel)
+are covered, each on the generic kernel too. The runtime
 dicts here are built over the raw arrays, without the descriptor gate, so
 that the below-gate directories reach the kernels.
 """
@@ -200,7 +201,7 @@ def _gemv_check(cuda, rt, expect, ms, what):
         assert planted is None or min(planted) > 1.0, f"{what} M={M}: a planted mistake passed ({planted})"
 
 
-@pytest.mark.parametrize("profile", ["sip", "gulp"])
+@pytest.mark.parametrize("profile", ["sip", "balanced", "gulp"])
 @pytest.mark.parametrize("C", [2048, 2100])
 def test_short_blocks_read_inside_the_pad(cuda, profile, C):
     from drinkme_amd import radix_ops

@@ -13,8 +13,7 @@ gate/up of a layer as one launch each, o and down alone).
     per CU, progress balance on);
   - the 32B-class layer (hidden 5120; q 8192x5120, k/v 1024x5120, o
     5120x8192, gate/up 25600x5120, down 5120x25600), Student-t(4) weights
-    scaled to std 0.02, gulp at M = 1 and M = 4 (the down projection at
-    M = 4 runs in column phases), and sip at M = 1.
+    scaled to std 0.02, gulp at M = 1 and M = 4, and sip at M = 1.
 
 The weights are the benchmark's own streams (drinkme_amd.synth), packed by
 the product encoder as bench.py packs them. Bars, as drinkme's gates put

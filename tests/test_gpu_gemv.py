@@ -236,9 +236,10 @@ def _gulp_bits(rng, kind, shape):
 @pytest.mark.parametrize("kind", ["normal", "t4", "spread", "terminal", "dense-tier1", "terminal-heavy", "long-tail"])
 @pytest.mark.parametrize("M", [1, 3, 8])
 def test_gulp_fast_path(cuda, kind, M):
-    """The gulp kernel (M = 1..8) across tier-1, tier-2 and terminal escape
-    densities, against the float64 bound and the generic kernel; with and
-    without the schedule in the descriptor."""
+    """gulp's GEMV (the wave kernel at M <= 4, the gulp kernel at 8) across
+    tier-1, tier-2 and terminal escape densities, against the float64 bound
+    and the generic kernel; with and without the schedule in the
+    descriptor."""
     import torch
 
     from drinkme_amd import radix_ops, swap

@@ -69,11 +69,9 @@ def test_group_matches_the_oracle(cuda, rows, C, M):
                                       ((8192, 1024, 1024), 5120, 1), ((12288, 12288), 4096, 1),
                                       ((640, 128, 128), 1024, 8), ((1000, 37, 2000), 2048, 1)])
 def test_gulp_group_matches_the_oracle(cuda, rows, C, M):
-    """gulp groups: the kernel keeps one tensor per workgroup, so q/k/v-like
-    groups run as one launch with a tile height that divides every tensor
-    boundary (8 rows for 4096/1024/1024: 768 tiles, so 8-wave workgroups,
-    three per CU, at M = 1, 2 and 4); a group with no such height
-    (1000/37/2000) runs tensor by tensor. Same bars as sip."""
+    """gulp groups: at M <= 4 one launch of the wave kernel, any row counts; at
+    8 the gulp kernel keeps one tensor per workgroup, with a tile height that
+    divides every tensor boundary. Same bars as sip."""
     import torch
 
     from drinkme_amd import radix_ops, swap
@@ -98,9 +96,10 @@ def test_gulp_group_matches_the_oracle(cuda, rows, C, M):
 
 
 def test_group_fallbacks_match_the_oracle(cuda):
-    """Groups the one-launch kernel does not take run tensor by tensor:
-    more than four tensors, a tensor shorter than the row tile, a gulp
-    member, M = 3, fp32 activations."""
+    """Groups the sip kernel does not take as one launch: more than four
+    tensors, a tensor shorter than the row tile and a gulp member run tensor by
+    tensor; fp32 activations one launch of the wave kernel where the profiles
+    agree. M = 1 and 3."""
     import torch
 
     from drinkme_amd import radix_ops, swap

@@ -5,12 +5,14 @@ the kernel the compressed tensor of its widths runs, with the decode
 replaced by a load of the raw weight at the same (row, column), so at any
 one launch plan the two outputs are identical.
 
-Covered: every profile (sip and gulp on their fast kernels, balanced on the
-generic one), M = 1..8, fp32 and bf16 outputs, the fused bias epilogue, a
-row long enough for column phases at M = 8, columns that are not a whole
-number of blocks (the generic kernel at every profile), an fp32
-activation (the generic kernel's widening path), and a 12288 x 4096
-launch long enough for the sip kernel's progress balance.
+Covered: every profile, M = 1..8, fp32 and bf16 outputs, the fused bias
+epilogue, whole blocks (sip on its kernel; gulp on the wave kernel at M <= 4
+and its own beyond; balanced on the wave kernel), columns that are not a whole
+number of blocks and an fp32 activation (the wave kernel at every profile), all
+of these on the generic kernel too; a row long enough for column phases at
+M = 8, rows past the wave kernel's LDS, and a 12288 x 4096 launch long enough
+for the sip kernel's progress balance. (gulp rows past the wave kernel's sums:
+tests/test_gpu_wave.py.)
 """
 
 import zlib
@@ -32,9 +34,18 @@ def _pair(bits, profile, cuda):
     return p, twin
 
 
+@pytest.fixture(params=["auto", "generic"])
+def policy(request):
+    from drinkme_amd import radix_ops
+
+    prev = radix_ops.set_policy(request.param)
+    yield request.param
+    radix_ops.set_policy(prev)
+
+
 @pytest.mark.parametrize("profile", ["sip", "gulp", "balanced"])
 @pytest.mark.parametrize("shape", [(512, 4096), (300, 3584), (1000, 2048)])
-def test_twin_is_its_compressed_tensor_bit_for_bit(cuda, profile, shape):
+def test_twin_is_its_compressed_tensor_bit_for_bit(cuda, profile, shape, policy):
     import torch
 
     from drinkme_amd import radix_ops
@@ -46,13 +57,13 @@ def test_twin_is_its_compressed_tensor_bit_for_bit(cuda, profile, shape):
     xb = O.f32_to_bf16_bits(rng.standard_normal((8, C)).astype(np.float32))
     x = bf16_tensor(xb, cuda)
     bias = bf16_tensor(O.f32_to_bf16_bits(rng.standard_normal(R).astype(np.float32)), cuda)
-    print(f"case twin {profile} {shape}", flush=True)
+    print(f"case twin {profile} {shape} {policy}", flush=True)
     assert torch.equal(radix_ops.gemv(twin, x[0]), radix_ops.gemv(p, x[0])), "gemv M=1"
     assert torch.equal(radix_ops.gemv_fused(twin, x[0], bias), radix_ops.gemv_fused(p, x[0], bias)), "fused"
     for M in range(2, 9):
         a, b = radix_ops.gemv_mc(twin, x[:M]), radix_ops.gemv_mc(p, x[:M])
         assert torch.equal(a, b), f"gemv_mc M={M}: max |diff| {(a - b).abs().max().item():.3g}"
-    # an fp32 activation: both run the generic kernel
+    # an fp32 activation: both run the wave kernel (or the generic one)
     xf = x[:3].float()
     assert torch.equal(radix_ops.gemv_mc(twin, xf), radix_ops.gemv_mc(p, xf)), "fp32 x"
     # and the twin is right, not only equal
@@ -63,8 +74,9 @@ def test_twin_is_its_compressed_tensor_bit_for_bit(cuda, profile, shape):
 
 @pytest.mark.parametrize("profile", ["sip", "gulp"])
 def test_twin_matches_through_column_phases(cuda, profile):
-    """M = 8 over 16384 columns needs 256 KB of activation rows: the fast
-    kernels run it in column phases, and the twin in the same phases."""
+    """M = 8 over 16384 columns needs 256 KB of activation rows: the sip and
+    gulp kernels run it in column phases, and the twin in the same phases (as
+    the sip kernel's at M = 4; gulp's M <= 4 is the wave kernel's, in one)."""
     import torch
 
     from drinkme_amd import radix_ops

@@ -110,13 +110,14 @@ def test_a_non_finite_weight_past_the_row_end_is_not_multiplied(cuda):
             assert np.all(np.isinf(y[:6])) and np.all(np.isfinite(y[6:])), profile
 
 
-@pytest.mark.parametrize("M,blocks", [(1, 2047), (1, 2049), (3, 512), (4, 513), (2, 4), (4, 1)])
+@pytest.mark.parametrize("M,blocks", [(1, 2047), (1, 2049), (2, 1025), (3, 512), (4, 513), (2, 4), (4, 1)])
 def test_gulp_rows_at_the_edge_of_the_wave_kernels_sums(cuda, M, blocks):
     """Whole-block gulp at up to four rows runs the wave kernel while two
     rows' sums fit it (2048 / M column blocks, M rounded up to a power of
     two), the gulp kernel beyond; three rows of weights, the second of the
-    last unit missing. The twin follows bit for bit, from a 16-byte-aligned
-    weight and from one that is not."""
+    last unit missing. The twin follows bit for bit on either side of the
+    edge, and on the wave kernel's from a weight that is not 16-byte aligned
+    too (the gulp kernel's twin needs that alignment)."""
     import torch
 
     from drinkme_amd import radix_ops, swap
@@ -131,13 +132,36 @@ def test_gulp_rows_at_the_edge_of_the_wave_kernels_sums(cuda, M, blocks):
     y = radix_ops.gemv_rows(rt, x, None, torch.float32)
     ref, bound = O.gemv_f64(bits, O.bf16_bits_to_f32(xb))
     assert np.all(np.abs(y.cpu().numpy().astype(np.float64) - ref) <= bound)
-    if blocks <= 512:  # (past that, the gulp kernel and its twin: test_gpu_twin)
-        buf = torch.empty(R * C + 2, dtype=torch.bfloat16, device=cuda)
-        for start in (0, 2):
-            w = buf[start:start + R * C].view(R, C)
-            w.copy_(bf16_tensor(bits, cuda))
-            twin = dict(swap.to_device_twin(w, widths=rt["widths"], device=cuda), weight=w)
-            assert torch.equal(radix_ops.gemv_rows(twin, x, None, torch.float32), y), start
+    buf = torch.empty(R * C + 2, dtype=torch.bfloat16, device=cuda)
+    for start in (0, 2) if blocks * (M if M < 3 else 4) <= 2048 else (0,):
+        w = buf[start:start + R * C].view(R, C)
+        w.copy_(bf16_tensor(bits, cuda))
+        twin = dict(swap.to_device_twin(w, widths=rt["widths"], device=cuda), weight=w)
+        assert torch.equal(radix_ops.gemv_rows(twin, x, None, torch.float32), y), start
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("profile", ["sip", "balanced", "gulp"])
+def test_the_generic_kernel_on_the_wave_kernels_tensors(cuda, profile, dtype):
+    """Other block sizes and rows past the wave kernel's sums still run it."""
+    import torch
+
+    from drinkme_amd import radix_ops, swap
+
+    for R, C in ((130, 260), (17, 3079), (64, 2048)):
+        rng = np.random.default_rng(R + C)
+        bits = finite_bits(rng, (R, C), spread=True)
+        rt = swap.to_device_radix(pack_to_dict(O.pack(bits, profile, allow_raw=False), profile), cuda)
+        x = torch.from_numpy(rng.standard_normal((8, C)).astype(np.float32)).to(cuda).to(getattr(torch, dtype))
+        ref, bound = O.gemv_f64(bits, x.float().cpu().numpy())
+        print(f"case wave generic {profile} {dtype} {(R, C)}", flush=True)
+        prev = radix_ops.set_policy("generic")
+        try:
+            for M in range(1, 9):
+                y = radix_ops.gemv_rows(rt, x[:M], None, torch.float32).cpu().numpy().astype(np.float64)
+                assert np.all(np.abs(y - ref[:M]) <= bound[:M]), f"{(R, C)} M={M}"
+        finally:
+            radix_ops.set_policy(prev)
 
 
 # (escapes of tier 0, of tier 1, of tier 2) of a block, by profile: none, the in-register tiers' limits (sip 256

@@ -211,6 +211,12 @@ void run(const Case& cs) {
         return;  // the generic kernel runs
     const bool dec = cs.kind == kDecodeSip || cs.kind == kDecodeGulp;
     if (dec && sh.phases > 1) return;  // the decode runs unphased, else generic
+    const bool gulp_rows = cs.kind == kGulp || cs.kind == kTwinGulp || cs.kind == kGulpMatrix || cs.kind == kTwinGulpMatrix;
+    if (gulp_rows && !l.quad) {  // the wave kernel's, but for the rows it leaves: those have a kernel for several phases
+        const uint32_t one = 1;
+        if (wave_plan(kWaveGulp, false, kWaveX16, M, &one, 1, sh.nb, cs.cus)) return;
+        if (sh.phases < 2) bad(describe(cs) + ": one phase, and neither kernel takes it");
+    }
     ++g_plans;
     const std::string tag = describe(cs);
     if ((lds + l.fixed) > kLdsBytes) bad(tag + ": LDS past the CU's");
@@ -371,7 +377,7 @@ int main(int argc, char** argv) {
         {{4096}, 4096},         {{4096, 1024, 1024}, 4096}, {{12288, 12288}, 4096}, {{4096}, 12288},
         {{151936}, 4096},       {{8192, 1024, 1024}, 5120}, {{5120}, 8192},          {{25600, 25600}, 5120},
         {{5120}, 25600},        {{1024}, 4096},             {{1}, 1024},             {{3, 5, 7, 9}, 2048},
-        {{1000, 24, 3000}, 3072}};
+        {{1000, 24, 3000}, 3072}, {{40}, 1024 * 2052},        {{3, 70}, 1024 * 1026},    {{17}, 1024 * 520}};
     const Kind kinds[] = {kSip, kGulp, kDecodeSip, kDecodeGulp, kTwinSip, kTwinGulp, kGulpMatrix, kTwinGulpMatrix};
     for (const auto& s : shapes)
         for (Kind k : kinds)
