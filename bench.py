@@ -76,6 +76,14 @@ def algorithmic_bytes(rt: dict, m: int = 1) -> int:
     return 4 * int(rt["NW"]) + 4 * (R * nb + 1) + PALETTE_BYTES[rt["profile"]] + 2 * m * C + 2 * m * R
 
 
+def kernel_of(profile: str, m: int) -> str:
+    """The kernel that AUTO runs for the workloads' launches (whole blocks,
+    bf16 activations; dmx_radix_gemv's routing)."""
+    if profile == "sip":
+        return "k_gemv_sip"
+    return "k_gemv_gulp" if profile == "gulp" and m > 4 else "k_gemv_wave"
+
+
 def workload_items(name: str):
     """(workload, layer, tensor, rows, cols, distribution) per GEMV."""
     from drinkme_amd import synth
@@ -455,7 +463,7 @@ def main() -> int:
     for name, pk in per_kind.items():
         log(f"  {name}: {pk['bytes'] / 1e6:.1f} MB, kernel {pk['kernel_us']:.2f} us, plain read {pk['read_us']:.2f} us "
             f"({pk['kernel_over_read']:.2f}x), {pk['launches']} launch(es) in its graph")
-    # gulp's 3- and 4-row verify: AUTO runs it on v_dot2 (measured faster);
+    # gulp's 3- and 4-row verify: AUTO runs it on v_dot2 (the wave kernel);
     # the matrix policy runs it in quad units on the matrix cores, as 8 rows
     # run: the same sweep timed on that path too
     matrix = None
@@ -508,7 +516,7 @@ def main() -> int:
         f"{total_bytes / (ms_md * 1e-3) / 1e9:.0f} GB/s compressed")
     traffic = None
     tf = os.path.join(ROOT, "profiles", "traffic.json")
-    key = f"k_gemv_{args.profile} {dom_shape} {args.profile} M={args.m}"
+    key = f"{kernel_of(args.profile, args.m)} {dom_shape} {args.profile} M={args.m}"
     if os.path.exists(tf):
         traffic = json.load(open(tf)).get(key, {}).get("hbm_bytes_per_launch")
     cpu = None
@@ -559,7 +567,7 @@ def main() -> int:
         "roofline": {
             "bound": "hbm", "achieved": round(achieved, 1), "peak": PEAK_GBPS, "unit": "GB/s",
             "frac": round(achieved / PEAK_GBPS, 4), "traffic": traffic,
-            "kernel": {"sip": "k_gemv_sip", "gulp": "k_gemv_gulp"}.get(args.profile, "k_gemv_generic"),
+            "kernel": kernel_of(args.profile, args.m),
             "shape": dom_shape,
             "bytes_per_launch": round(dom_bytes), "us_per_launch": round(dom_us, 3),
             "launches_timed": len(dom), "settle_replays": dom_info["settle_replays"],

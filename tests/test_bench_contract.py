@@ -43,6 +43,16 @@ def test_algorithmic_bytes_is_the_stated_formula():
     assert bench.algorithmic_bytes(rt, 4) == 4 * 1234 + 4 * (3 * nb + 1) + 21 + 2 * 4 * 2100 + 2 * 4 * 3
 
 
+def test_the_line_names_the_kernel_that_runs():
+    assert [bench.kernel_of("sip", m) for m in (1, 4, 8)] == ["k_gemv_sip"] * 3
+    assert [bench.kernel_of("gulp", m) for m in (1, 4, 5, 8)] == ["k_gemv_wave"] * 2 + ["k_gemv_gulp"] * 2
+    assert [bench.kernel_of("balanced", m) for m in (1, 8)] == ["k_gemv_wave"] * 2
+    # and the measured bytes it looks up are that kernel's
+    for key in json.load(open(os.path.join(ROOT, "profiles", "traffic.json"))):
+        kernel, *_, profile, m = key.split(" ")
+        assert kernel == bench.kernel_of(profile, int(m.split("=")[1])), key
+
+
 def test_workloads_hold_the_configured_gemvs():
     step = bench.workload_items("qwen3-8b-step")
     assert len(step) == 36 * 7 + 1 and step[-1][3:5] == (151936, 4096)
