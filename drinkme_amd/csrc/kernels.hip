@@ -2362,7 +2362,6 @@ int launch_wave(int p, bool raw, const dmx_radix_tensor* const* ts, uint32_t n, 
     sh.cols = ts[0]->cols;
     sh.nb = (sh.cols + 1023) / 1024;
     sh.m = m;
-    sh.x_dtype = x_dtype;
     sh.bias_dtype = bias_dtype;
     sh.out_dtype = out_dtype;
     sh.wide = xt == kWaveX32 || (sh.cols % 2 == 0 && reinterpret_cast<uintptr_t>(x) % 4 == 0);

@@ -17,9 +17,11 @@
 //
 // What bounds it: for launches of a few units a wave, the 6 us before and
 // after them (the directory's round trip, the first payload, the tables);
-// for longer ones the payload's stream and the VALU (76 instructions a sip
-// block at M = 1 bf16, 88 to 98 with more tiers, 16 M + 16 more for fp32
-// products). Measured, one launch, against k_gemv_generic, which scans over
+// for longer ones the decode: the VALU is busy 65% of the time (gulp, M = 1,
+// 2 x 12288 x 4096; 70% at M = 4), 105 instructions a block (143) beside 60
+// scalar and 18 LDS ones, and of a wave's life 37% issues (36%), 35% waits on a
+// dependency (32%) and 28% for an issue slot (32%). (fp32 products are 16 M +
+// 16 instructions a block more.) Measured, one launch, against k_gemv_generic, which scans over
 // a workgroup with two barriers a tier: sip 2 x 9472 x 3584 (ragged) 21.2 us
 // for 284, sip 3584 x 9472 14.3 for 149; gulp fp32 M = 2 q/k/v of 10240 x
 // 5120 23.8 for 326; balanced q/k/v of 6144 x 4096 12.8 for 145. Against
@@ -590,7 +592,7 @@ struct WaveShape {
     uint32_t tile;  // T: rows per workgroup, even
     uint32_t m;     // activation rows (<= the kernel's M; the rest repeat the last one)
     uint32_t wide;  // 1: x's rows (raw: the weight's too) may be read four bytes at a time
-    int x_dtype, bias_dtype, out_dtype;
+    int bias_dtype, out_dtype;
 };
 
 struct __attribute__((packed, aligned(4))) Quad4 {
